@@ -21,7 +21,7 @@ enum HopFlags {
   HOP_NT_STORE = 1,       // streaming (non-temporal) stores of the output
   HOP_NO_XCD_REMAP = 2,   // keep the hardware block order
   HOP_SPATIAL = 4,        // XCD x owns spatial block x of the lattice (all rhs),
-                          // swept along t (Wilson kind, needs the XCD remap)
+                          // swept along t (needs the XCD remap)
   HOP_SITEWAVE = 8,       // a wavefront computes one site for 64/nb rhs (Wilson
                           // kind, nb divides 64, no partials): the site's
                           // neighbour entries and links are wave-uniform
@@ -38,6 +38,9 @@ enum HopFlags {
                           // the 16 lanes of a DPP row (one site's slots) load
                           // one 4-byte word of each link each and exchange
                           // them by row broadcasts
+  HOP_QUAD = 512,         // half-precision spinors, 18-real links, nb a multiple
+                          // of 4: the SU(3) products on the matrix cores, four
+                          // slots of a site per 4x4 block (hop_quad.hip)
 };
 inline int hop_rhsgroup_G(int flags) { return (flags & HOP_RHSGROUP) ? (2 << ((flags >> 6) & 3)) : 1; }
 
@@ -94,13 +97,18 @@ struct HopParams {
   const int* ractive;
   const uint4* nbr;         // neighbour table (k_build_nbr)
   const uint32_t* nbr_neg;
-  // HOP_SPATIAL: site_cb of logical site b*perm_S + q (the same table for
-  // both parities), perm_S = Vcb / 8 sites per spatial block
+  // HOP_SPATIAL: site of logical site b*perm_S + q, perm_S sites per spatial
+  // block: Wilson kind site_cb (the same table for both parities), perm_S =
+  // Vcb / 8; DWF kind parity*Vcb + site_cb, both parities of a slice after
+  // one another, perm_S = Vcb / 4
   const uint32_t* perm;
   int perm_S;
   // launch geometry set by the launcher for the chosen block size: blocks
   // per rhs, blocks per (spatial block, rhs), log2(nb) or -1
   int bpr, bpr_b, nb_shift;
+  // HOP_QUAD: multiplier and shift of the division by nb (set by the launcher)
+  uint32_t nb_magic;
+  int nb_mshift;
   // HOP_LDS_LINKS: sites per block the LDS area is sized for (set by the
   // launcher)
   int lds_sites;
@@ -142,6 +150,8 @@ enum { CLOV_NONE = 0, CLOV_POST = 1, CLOV_X = 2, CLOV_S5X = 3, CLOV_S5XR = 4, CL
 hipError_t launch_hop(const HopParams& P, hipStream_t st);
 hipError_t build_nbr(const Geom& g, uint4* nbr, uint32_t* nbr_neg, hipStream_t st);
 hipError_t launch_hop_clover(const HopParams& P, hipStream_t st);
+hipError_t launch_hop_quad(const HopParams& P, hipStream_t st);
+hipError_t pack_gauge_quad(bool bf16, const double* aos, void* out, const uint4* nbr, int Vcb, hipStream_t st);
 
 // link storage read by a hop precision
 inline int link_storage_of(int hprec) {
@@ -198,6 +208,21 @@ inline bool link_row_setup(const HopParams& Q, int bs) {
   if (!half || Q.kind != KIND_WILSON || Q.nb != 16 || bs % 16) return false;
   if (Q.flags & (HOP_SITEWAVE | HOP_LDS_LINKS | HOP_RHSGROUP)) return false;
   return Q.gauge.plane * 16 * 3 < (int64_t(1) << 32);
+}
+
+// HOP_QUAD: whether the launch shape allows it at block size bs.  Four slots
+// of a site per group of 4 lanes and whole wavefronts (a matrix instruction
+// reads the link rows of all 4 lanes of a group); 24-bit products for the
+// element offsets (site < 2^24, 16 nb < 2^24) and 32-bit ones.  A mass per
+// rhs and the clover epilogues have no such kernel.
+inline bool quad_setup(const HopParams& Q, int bs) {
+  if (Q.prec != PREC_H_H18 && Q.prec != PREC_H_B18) return false;
+  if (Q.nb < 4 || Q.nb % 4 || Q.nb >= (1 << 20) || bs % 64) return false;
+  if (Q.geom.Vcb >= (1 << 24) || ((int64_t)Q.nsites_out * Q.nb) % bs) return false;
+  if ((int64_t)Q.nrhs * Q.nsites_out * Q.nb >= (int64_t(1) << 28)) return false;
+  if (Q.flags & (HOP_SITEWAVE | HOP_LDS_LINKS | HOP_RHSGROUP | HOP_LINK_ROW)) return false;
+  if (Q.clov == CLOV_NONE) return !Q.rupd || Q.kind == KIND_DWF;
+  return Q.clov == CLOV_S5X && (Q.hc5 == 0.0 || 64 % Q.nb == 0);
 }
 
 // block size dividing n (a power of two, at most 256)

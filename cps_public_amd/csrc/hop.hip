@@ -99,6 +99,7 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
 }
 
 hipError_t launch_hop(const HopParams& P, hipStream_t st) {
+  if (P.flags & HOP_QUAD) return launch_hop_quad(P, st);
   if (P.clov != CLOV_NONE && P.clov != CLOV_KS) return launch_hop_clover(P, st);
   switch (P.prec) {
     case PREC_D_D18: return launch_t<SpinD, SpinD, LinkD18, double>(P, st);

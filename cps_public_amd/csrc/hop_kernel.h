@@ -623,7 +623,7 @@ __device__ __forceinline__ HopElem hop_decode(const HopParams& P, int64_t sb64, 
   HopElem E;
   const int sb = (int)sb64, nsub = (int)nsub64;
   const int el_base = threadIdx.x;
-  if (KIND == KIND_WILSON && (P.flags & HOP_SPATIAL)) {
+  if (P.flags & HOP_SPATIAL) {
     // sb = (spatial block b = XCD, rhs, sub-block within (b, rhs))
     const int per_b = nsub >> 3;
     const int b = sb / per_b;
@@ -666,7 +666,7 @@ __device__ __forceinline__ void lds_fill_links(const HopParams& P, const HopElem
   const int sl = t >> 3, d = t & 7, mu = d & 3;
   const int q = E.qb + sl;
   const Geom& g = P.geom;
-  const int site = (KIND == KIND_WILSON && (P.flags & HOP_SPATIAL)) ? (int)P.perm[(int64_t)E.b * P.perm_S + q] : q;
+  const int site = (P.flags & HOP_SPATIAL) ? (int)P.perm[(int64_t)E.b * P.perm_S + q] : q;
   int out_par, site_cb;
   if (KIND == KIND_DWF) {
     out_par = site >= g.Vcb ? 1 : 0;

@@ -5,7 +5,9 @@
 namespace cpship {
 
 enum SpinStorage { STORE_D = 0, STORE_F = 1, STORE_H = 2 };
-enum LinkStorage { LINK_D18 = 0, LINK_F12 = 1, LINK_H12 = 2, LINK_B12 = 3, LINK_H18 = 4, LINK_B18 = 5, NLINK = 6 };
+enum LinkStorage { LINK_D18 = 0, LINK_F12 = 1, LINK_H12 = 2, LINK_B12 = 3, LINK_H18 = 4, LINK_B18 = 5,
+                   LINK_HQ = 6, LINK_BQ = 7,   // the links onto each site together (pack_gauge_quad)
+                   NLINK = 8 };
 enum SpinMap { MAP_4D = 0, MAP_DWF5 = 1, MAP_4DPREC = 2 };
 
 hipError_t pack_spinor(int storage, const double* aos, const FieldRef& out, int map, int Vcb, int ls, int cb5,

@@ -585,10 +585,6 @@ static int hop4(Lattice& L, int hprec, const FieldRef& out, const FieldRef& in, 
     P.m5b = m5->b;
     P.m5c = m5->c;
   }
-  const int lstore = link_storage_of(hprec);
-  int rc = L.ensure_gauge(lstore);
-  if (rc) return rc;
-  P.gauge = L.gauge_ref(lstore);
   return tuned_launch(L, P);
 }
 

@@ -85,9 +85,10 @@ struct Lattice {
   std::vector<Field> scratch;
   DevBuf partial, scal, io, io2;
   DevBuf nbr, nbr_neg;   // neighbour table of the geometry (hop kernels)
-  // spatial site order of the HOP_SPATIAL launches (built on first use):
-  // 0 not built, 1 built, -1 the geometry has no 8-way (y, z) split
-  DevBuf perm;
+  // spatial site order of the HOP_SPATIAL launches (built on first use),
+  // perm for one parity and perm5 for both (DWF fields): 0 not built, 1
+  // built, -1 the geometry has no 8-way (y, z) split
+  DevBuf perm, perm5;
   int perm_state = 0;
   int ensure_perm();
   // clover sets [kappa][cb] (cb 0: A_ee^-1, cb 1: A_oo) per storage format;

@@ -205,6 +205,15 @@ int Lattice::set_hop_phase(HopParams& P, int hprec) const {
 int Lattice::ensure_gauge(int link_storage) {
   if (gauge_valid[link_storage]) return 0;
   const int64_t plane = (int64_t)8 * g.Vcb;
+  if (link_storage == LINK_HQ || link_storage == LINK_BQ) {
+    // 8 links of 36 bytes per output site, each stored with both its ends
+    const int qrc = gauge[link_storage].ensure((size_t)plane * 2 * 36);
+    if (qrc) return qrc;
+    CPSHIP_CHECK(pack_gauge_quad(link_storage == LINK_BQ, (const double*)gauge_aos.p, gauge[link_storage].p,
+                                 (const uint4*)nbr.p, g.Vcb, stream));
+    gauge_valid[link_storage] = true;
+    return 0;
+  }
   int rc = gauge[link_storage].ensure((size_t)plane * link_bytes(link_storage));
   if (rc) return rc;
   GaugeRef gr;
@@ -257,6 +266,18 @@ int Lattice::ensure_perm() {
   int rc = perm.ensure(h.size() * sizeof(uint32_t));
   if (rc) return rc;
   CPSHIP_CHECK(hipMemcpy(perm.p, h.data(), h.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  if (ls > 1) {
+    // both parities of a block's slice after one another
+    std::vector<uint32_t> h5(2 * h.size());
+    const size_t slice = (size_t)lh * ny * nz;
+    for (size_t k = 0; k < h.size() / slice; k++)
+      for (size_t i = 0; i < slice; i++) {
+        h5[2 * k * slice + i] = h[k * slice + i];
+        h5[(2 * k + 1) * slice + i] = (uint32_t)g.Vcb + h[k * slice + i];
+      }
+    if ((rc = perm5.ensure(h5.size() * sizeof(uint32_t)))) return rc;
+    CPSHIP_CHECK(hipMemcpy(perm5.p, h5.data(), h5.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  }
   perm_state = 1;
   return 0;
 }
@@ -355,10 +376,6 @@ int hop_ex(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& out, con
   P.in = in;
   P.out = out;
   P.X = X;
-  int lstore = link_storage_of(hprec);
-  rc = L.ensure_gauge(lstore);
-  if (rc) return rc;
-  P.gauge = L.gauge_ref(lstore);
   P.partial = partial;
   if (hc) {
     P.clov = hc->mode;
@@ -460,8 +477,8 @@ static bool tuning_enabled() { return knob(&cps_hip_tuning::tune, "CPS_HIP_TUNE"
 
 // whether a launch may use HOP_SPATIAL at block size b
 static bool spatial_ok(Lattice& L, const HopParams& P, int b) {
-  if (P.kind != KIND_WILSON || L.g.Vcb % 8) return false;
-  const long long per_b = (long long)(L.g.Vcb / 8) * P.nb;
+  if (L.g.Vcb % 8) return false;
+  const long long per_b = (long long)(L.g.Vcb / 8) * P.nb * (P.kind == KIND_DWF ? 2 : 1);
   if (per_b % b) return false;
   return L.ensure_perm() == 0;
 }
@@ -506,9 +523,27 @@ int tuned_launch(Lattice& L, HopParams& P) {
   P.nbr = (const uint4*)L.nbr.p;
   P.nbr_neg = (const uint32_t*)L.nbr_neg.p;
   P.perm = nullptr;
-  P.perm_S = L.g.Vcb / 8;
+  P.perm_S = P.kind == KIND_DWF ? L.g.Vcb / 4 : L.g.Vcb / 8;
   const long long per_rhs = (long long)P.nsites_out * P.nb;
   const int def_block = pick_block(per_rhs);
+  // hop_mode: the field, or CPS_HIP_HOP_MODE=element|sitewave|lds|rhsgroup|row
+  int mode;
+  {
+    std::lock_guard<std::mutex> lk(tuning_mu);
+    mode = tuning_fields.hop_mode;
+  }
+  if (const char* m = getenv("CPS_HIP_HOP_MODE"))
+    mode = !strcmp(m, "sitewave") ? 2 : !strcmp(m, "element") ? 1 : !strcmp(m, "lds") ? 3 : !strcmp(m, "rhsgroup") ? 4
+         : !strcmp(m, "row") ? 5 : 0;
+  // half precision with a multiple of 4 slots per site: the matrix-core
+  // kernel wherever the shape allows it, unless another mapping is asked for
+  P.flags = 0;
+  const bool quad = mode == 0 && !tl_no_alloc && quad_setup(P, def_block);
+  {
+    const int lstore = quad ? (P.prec == PREC_H_B18 ? LINK_BQ : LINK_HQ) : link_storage_of(P.prec);
+    if (int rc = L.ensure_gauge(lstore)) return rc;
+    P.gauge = L.gauge_ref(lstore);
+  }
   if (tl_no_alloc) {
     // no allocation and no timing (cps_hip_matpc_dag_matpc_noalloc): the
     // choice cached for this launch shape if it needs no table the handle
@@ -534,8 +569,8 @@ int tuned_launch(Lattice& L, HopParams& P) {
     CPSHIP_CHECK(launch_hop(P, L.stream));
     return 0;
   }
-  if (P.kind == KIND_WILSON && L.perm_state >= 0 && L.g.Vcb % 8 == 0 && L.ensure_perm() == 0)
-    P.perm = (const uint32_t*)L.perm.p;
+  if (L.perm_state >= 0 && L.g.Vcb % 8 == 0 && L.ensure_perm() == 0)
+    P.perm = (const uint32_t*)(P.kind == KIND_DWF ? L.perm5.p : L.perm.p);
   if (P.clov == CLOV_KS) {
     // a mass per rhs: one kernel in element order (no variants to time)
     P.block = def_block;
@@ -543,17 +578,8 @@ int tuned_launch(Lattice& L, HopParams& P) {
     CPSHIP_CHECK(launch_hop(P, L.stream));
     return 0;
   }
-  // hop_mode: the field, or CPS_HIP_HOP_MODE=element|sitewave|lds|rhsgroup|row
-  int mode;
-  {
-    std::lock_guard<std::mutex> lk(tuning_mu);
-    mode = tuning_fields.hop_mode;
-  }
-  if (const char* m = getenv("CPS_HIP_HOP_MODE"))
-    mode = !strcmp(m, "sitewave") ? 2 : !strcmp(m, "element") ? 1 : !strcmp(m, "lds") ? 3 : !strcmp(m, "rhsgroup") ? 4
-         : !strcmp(m, "row") ? 5 : 0;
   HopTuneKey key{P.kind, P.prec, P.dag, P.nb, P.nsites_out, P.nrhs, P.partial != nullptr, P.X.data != nullptr,
-                 P.clov + 16 * P.m5post + 32 * P.rupd, {L.g.L[0], L.g.L[1], L.g.L[2], L.g.L[3]}, mode};
+                 P.clov + 16 * P.m5post + 32 * P.rupd, {L.g.L[0], L.g.L[1], L.g.L[2], L.g.L[3]}, mode + (quad ? 16 : 0)};
   HopTuneVal chosen;
   bool have = false;
   {
@@ -592,7 +618,9 @@ int tuned_launch(Lattice& L, HopParams& P) {
     // order: 6.2 against 4.6 ms for the 32^3x64 clover hop with 48 rhs); with
     // per-chunk partials the element order is the default and the rhs-group
     // mapping a candidate
-    HopTuneVal best{def_block, (P.nb >= 8 && spatial_ok(L, P, def_block)) ? HOP_SPATIAL : 0, 0.0};
+    HopTuneVal best{def_block, (P.nb >= 8 && P.kind == KIND_WILSON && spatial_ok(L, P, def_block)) ? HOP_SPATIAL : 0,
+                    0.0};
+    if (quad) best.flags = HOP_QUAD | (spatial_ok(L, P, def_block) ? HOP_SPATIAL : 0);
     // a launch that updates a field in place (rupd) is never timed on the
     // live data: it keeps the fixed order of launches with partials
     if (tuning_enabled() && !P.rupd) {
@@ -610,10 +638,12 @@ int tuned_launch(Lattice& L, HopParams& P) {
       // stores, then the row-shared links with the order variants (tried
       // with CPS_HIP_HOP_MODE=row only)
       std::vector<int> cand;
-      for (int f = 0; f < 32; f++) cand.push_back(f);
-      for (int g = 0; g < 4; g++)
+      if (quad)
+        cand = {HOP_QUAD, HOP_QUAD | HOP_NO_XCD_REMAP, HOP_QUAD | HOP_SPATIAL};
+      for (int f = 0; f < 32 && !quad; f++) cand.push_back(f);
+      for (int g = 0; g < 4 && !quad; g++)
         for (int nt = 0; nt < 2; nt++) cand.push_back(HOP_RHSGROUP | (g << 6) | nt);
-      for (int f = 0; f < 8; f++) cand.push_back(HOP_LINK_ROW | f);
+      for (int f = 0; f < 8 && !quad; f++) cand.push_back(HOP_LINK_ROW | f);
       for (int b : blocks)
         for (int f : cand) {
           {
@@ -631,6 +661,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
               continue;
             }
           }
+          if (quad && !quad_setup(P, b)) continue;
           if (f & HOP_RHSGROUP) {
             if (!rhsgroup_ok(P, b, f) || mode == 1 || mode == 2 || mode == 3) continue;
           } else if (mode == 4 && (rhsgroup_ok(P, b, HOP_RHSGROUP) || rhsgroup_ok(P, def_block, HOP_RHSGROUP))) {
