@@ -38,9 +38,9 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
     return hipErrorInvalidValue;
   if (P.rupd) {
     // the CG residual update instead of the store (CLOV_NRR): half-precision
-    // DWF hops with X, element order, no variants
+    // DWF hops with X, element or spatial order, no variants
     if (P.clov != CLOV_NONE || P.kind != KIND_DWF || !P.X.data || !P.R.data || !P.ralpha || !P.ractive || P.m5post ||
-        (P.flags & (HOP_SPATIAL | HOP_SITEWAVE | HOP_LDS_LINKS | HOP_RHSGROUP | HOP_LINK_ROW)))
+        (P.flags & (HOP_SITEWAVE | HOP_LDS_LINKS | HOP_RHSGROUP | HOP_LINK_ROW)))
       return hipErrorInvalidValue;
     if constexpr (std::is_same<SIN, SpinH>::value) {
       if (P.dag) {

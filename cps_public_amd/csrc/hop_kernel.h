@@ -97,6 +97,19 @@ __device__ __forceinline__ void su3_dag_mul(const cplx<R> u[9], const cplx<R> h[
     }
 }
 
+// Direction that a kernel takes k-th.  A site of the two outputs' x line is
+// +x neighbour of one and -x neighbour of the other (and likewise along y in
+// the next line), so the loads of +mu and -mu meet in the vector L1 when they
+// follow each other closely; with all +mu before all -mu the FP64 hop fetches
+// every neighbour 8 times from L2.  4-D kind: +mu, -mu in turn (FP64 Wilson
+// hop of 16^3x32, 12 rhs, 131 -> 115 us; +x +y -x -y ..: 121).  Domain-wall
+// kind, whose sites are 8 lanes wide: +x +y -x -y, +z +t -z -t (FP64,
+// 16^3x32, Ls 16: 189 -> 166 us; the other order 170).
+template <int KIND>
+__host__ __device__ constexpr int hop_dir(int k) {
+  return KIND == KIND_DWF ? (k & 1) + (k & 2) * 2 + (k & 4) / 2 : (k >> 1) + 4 * (k & 1);
+}
+
 struct Coord {
   int x[4];
 };
@@ -392,7 +405,7 @@ __device__ __forceinline__ void dir_compute(const SpinRaw<SIN>& sr, const LinkRa
 
 // Directions D0 .. D0+NB-1: all their spinor and link loads are issued
 // before the first of them is decoded.
-template <int D0, int NB, typename SIN, typename LK, typename R, int DAG>
+template <int D0, int NB, typename SIN, typename LK, typename R, int DAG, int KIND>
 __device__ __forceinline__ void hop_batch(const HopParams& P, const Nbr& N, int out_par, int site_cb,
                                           int64_t in_base, int j, cplx<R> acc[12]) {
   const int Vcb = P.geom.Vcb;
@@ -400,7 +413,7 @@ __device__ __forceinline__ void hop_batch(const HopParams& P, const Nbr& N, int 
   LinkRaw<LK> lr[NB];
 #pragma unroll
   for (int k = 0; k < NB; k++) {
-    const int d = D0 + k;
+    const int d = hop_dir<KIND>(D0 + k);
     raw_load<SIN>(sr[k], P.in, in_base + (int64_t)N.idx[d] * P.nb + j);
     const int mu = d & 3;
     const int64_t lidx = (d < 4) ? (int64_t)(out_par * 4 + mu) * Vcb + site_cb
@@ -409,28 +422,28 @@ __device__ __forceinline__ void hop_batch(const HopParams& P, const Nbr& N, int 
   }
 #define CPSHIP_DIR(K)                                                                             \
   if constexpr ((K) < NB) {                                                                       \
-    const float2 ph = link_phase(P, N.neg, D0 + (K));                                             \
-    dir_compute<D0 + (K), SIN, LK, R, DAG>(sr[K], lr[K], ph, acc);                                \
+    const float2 ph = link_phase(P, N.neg, hop_dir<KIND>(D0 + (K)));                                             \
+    dir_compute<hop_dir<KIND>(D0 + (K)), SIN, LK, R, DAG>(sr[K], lr[K], ph, acc);                                \
   }
   CPSHIP_DIR(0) CPSHIP_DIR(1) CPSHIP_DIR(2) CPSHIP_DIR(3) CPSHIP_DIR(4) CPSHIP_DIR(5) CPSHIP_DIR(6) CPSHIP_DIR(7)
 #undef CPSHIP_DIR
 }
 
 // HOP_LDS_LINKS: the spinor loads of directions D0 .. D0+NB-1 ...
-template <int D0, int NB>
+template <int D0, int NB, int KIND>
 __device__ __forceinline__ void hop_lds_load(const HopParams& P, const Nbr& N, int64_t in_base, int j,
                                              SpinRaw<SpinH> sr[NB]) {
 #pragma unroll
-  for (int k = 0; k < NB; k++) raw_load<SpinH>(sr[k], P.in, in_base + (int64_t)N.idx[D0 + k] * P.nb + j);
+  for (int k = 0; k < NB; k++) raw_load<SpinH>(sr[k], P.in, in_base + (int64_t)N.idx[hop_dir<KIND>(D0 + k)] * P.nb + j);
 }
 
 // ... and their products with the links staged in LDS (block site sl)
-template <int D0, int NB, int DAG>
+template <int D0, int NB, int DAG, int KIND>
 __device__ __forceinline__ void hop_lds_compute(const HopParams& P, const uint32_t* lds, int sl,
                                                 const SpinRaw<SpinH> sr[NB], cplx<float> acc[12]) {
 #define CPSHIP_DIR(K)                                                                             \
   if constexpr ((K) < NB) {                                                                       \
-    constexpr int D = D0 + (K);                                                                   \
+    constexpr int D = hop_dir<KIND>(D0 + (K));                                                                 \
     const uint4* w = reinterpret_cast<const uint4*>(lds + sl * LDS_SITE_WORDS + 8 * D);           \
     const uint4 a = w[0], b = w[1];                                                               \
     const uint32_t U[9] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w,                                \
@@ -784,7 +797,7 @@ __device__ __forceinline__ LinkRaw<LK> link_from_row(uint32_t v) {
 }
 
 // hop_batch with the links of HOP_LINK_ROW (half-precision spinors)
-template <int D0, int NB, typename LK, int DAG>
+template <int D0, int NB, typename LK, int DAG, int KIND>
 __device__ __forceinline__ void hop_batch_row(const HopParams& P, const Nbr& N, int out_par, int site_cb,
                                               int64_t in_base, int j, uint32_t loff, uint32_t lstride,
                                               cplx<float> acc[12]) {
@@ -793,7 +806,7 @@ __device__ __forceinline__ void hop_batch_row(const HopParams& P, const Nbr& N, 
   uint32_t lw[NB];
 #pragma unroll
   for (int k = 0; k < NB; k++) {
-    const int d = D0 + k;
+    const int d = hop_dir<KIND>(D0 + k);
     raw_load<SpinH>(sr[k], P.in, in_base + (int64_t)N.idx[d] * P.nb + j);
     const int mu = d & 3;
     const uint32_t lidx = (d < 4) ? (uint32_t)((out_par * 4 + mu) * Vcb + site_cb)
@@ -802,10 +815,10 @@ __device__ __forceinline__ void hop_batch_row(const HopParams& P, const Nbr& N, 
   }
 #define CPSHIP_DIR(K)                                                                             \
   if constexpr ((K) < NB) {                                                                       \
-    const float2 ph = link_phase(P, N.neg, D0 + (K));                                             \
+    const float2 ph = link_phase(P, N.neg, hop_dir<KIND>(D0 + (K)));                                             \
     uint32_t U[9];                                                                                \
     link_words_f16<LK>(link_from_row<LK>(lw[K]), ph, U);                                          \
-    dir_compute_h2w<D0 + (K), DAG>(sr[K], U, acc);                                                \
+    dir_compute_h2w<hop_dir<KIND>(D0 + (K)), DAG>(sr[K], U, acc);                                                \
   }
   CPSHIP_DIR(0) CPSHIP_DIR(1) CPSHIP_DIR(2) CPSHIP_DIR(3) CPSHIP_DIR(4) CPSHIP_DIR(5) CPSHIP_DIR(6) CPSHIP_DIR(7)
 #undef CPSHIP_DIR
@@ -924,14 +937,14 @@ __device__ __forceinline__ double hop_element(const HopParams& P, const HopElem&
     // the spinor loads go out before the block waits for its links
     constexpr int NBL = CPSHIP_HOP_BATCH_LDS;
     SpinRaw<SpinH> sr[NBL];
-    if (valid) hop_lds_load<0, NBL>(P, N, in_base, j, sr);
+    if (valid) hop_lds_load<0, NBL, KIND>(P, N, in_base, j, sr);
     lds_fill_links<LK, KIND>(P, E, lds);
     __syncthreads();
     if (valid) {
-      hop_lds_compute<0, NBL, DAG>(P, lds, E.sl, sr, acc);
+      hop_lds_compute<0, NBL, DAG, KIND>(P, lds, E.sl, sr, acc);
       if constexpr (NBL == 4) {
-        hop_lds_load<4, 4>(P, N, in_base, j, sr);
-        hop_lds_compute<4, 4, DAG>(P, lds, E.sl, sr, acc);
+        hop_lds_load<4, 4, KIND>(P, N, in_base, j, sr);
+        hop_lds_compute<4, 4, DAG, KIND>(P, lds, E.sl, sr, acc);
       }
     }
   }
@@ -940,28 +953,28 @@ __device__ __forceinline__ double hop_element(const HopParams& P, const HopElem&
     if constexpr (ROWL && std::is_same<SIN, SpinH>::value) {
       uint32_t loff, lstride;
       link_row_addr<LK>(P.gauge, j, loff, lstride);
-      hop_batch_row<0, 4, LK, DAG>(P, N, out_par, site_cb, in_base, j, loff, lstride, acc);
-      hop_batch_row<4, 4, LK, DAG>(P, N, out_par, site_cb, in_base, j, loff, lstride, acc);
+      hop_batch_row<0, 4, LK, DAG, KIND>(P, N, out_par, site_cb, in_base, j, loff, lstride, acc);
+      hop_batch_row<4, 4, LK, DAG, KIND>(P, N, out_par, site_cb, in_base, j, loff, lstride, acc);
     } else if constexpr (NB == 0) {
     } else if constexpr (NB == 8) {
-      hop_batch<0, 8, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<0, 8, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
     } else if constexpr (NB == 4) {
-      hop_batch<0, 4, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<4, 4, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<0, 4, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<4, 4, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
     } else if constexpr (NB == 2) {
-      hop_batch<0, 2, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<2, 2, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<4, 2, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<6, 2, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<0, 2, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<2, 2, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<4, 2, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<6, 2, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
     } else {
-      hop_batch<0, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<1, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<2, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<3, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<4, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<5, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<6, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
-      hop_batch<7, 1, SIN, LK, R, DAG>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<0, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<1, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<2, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<3, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<4, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<5, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<6, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
+      hop_batch<7, 1, SIN, LK, R, DAG, KIND>(P, N, out_par, site_cb, in_base, j, acc);
     }
 
     if constexpr (KIND == KIND_DWF) {

@@ -618,7 +618,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
     // order: 6.2 against 4.6 ms for the 32^3x64 clover hop with 48 rhs); with
     // per-chunk partials the element order is the default and the rhs-group
     // mapping a candidate
-    HopTuneVal best{def_block, (P.nb >= 8 && P.kind == KIND_WILSON && spatial_ok(L, P, def_block)) ? HOP_SPATIAL : 0,
+    HopTuneVal best{def_block, (P.nb >= 8 && spatial_ok(L, P, def_block)) ? HOP_SPATIAL : 0,
                     0.0};
     if (quad) best.flags = HOP_QUAD | (spatial_ok(L, P, def_block) ? HOP_SPATIAL : 0);
     // a launch that updates a field in place (rupd) is never timed on the
