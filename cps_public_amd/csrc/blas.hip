@@ -418,63 +418,81 @@ __global__ void __launch_bounds__(256) k_zero(FieldRef x, int64_t per_rhs) {
 }
 
 // One block per rhs: out[rhs] = sum of that rhs's partials (fixed order),
-// then the CG scalar step selected by mode.
-__global__ void k_reduce_rhs(const double* partial, int bpr, double* out, int mode, CGScalars cg) {
+// then the CG scalar step selected by mode.  Bound by latency: a thread adds
+// four partials per step, so that their loads overlap, the block is as wide
+// as the partials fill (reduce_threads), and the scalars are loaded before
+// the sum they are combined with.
+constexpr int REDUCE_MAX = 1024;
+
+__global__ void __launch_bounds__(REDUCE_MAX) k_reduce_rhs(const double* partial, int bpr, double* out, int mode,
+                                                           CGScalars cg) {
   const int rhs = blockIdx.x;
-  __shared__ double red[256];
-  double s = 0.0;
-  for (int k = threadIdx.x; k < bpr; k += blockDim.x) s += partial[(int64_t)rhs * bpr + k];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = blockDim.x >> 1; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+  __shared__ double red[REDUCE_MAX / 64];
+  const int was_active = (mode == RED_CG_ALPHA || mode == RED_CG_BETA) ? cg.active[rhs] : 0;
+  const int iters = (mode == RED_CG_ALPHA || mode == RED_CG_BETA) ? cg.iters[rhs] : 0;
+  const double old_rr = mode == RED_CG_ALPHA ? cg.rr[rhs] : 0.0;
+  const double old_alpha = mode == RED_CG_ALPHA ? cg.alpha[rhs] : 0.0;
+  const double stp = (mode == RED_CG_BETA || mode == RED_CG_INIT) ? cg.stp[rhs] : 0.0;
+  const double rr_prev = mode == RED_CG_BETA ? cg.rr_prev[rhs] : 0.0;
+  const double rr_upd = (mode == RED_CG_BETA && cg.rr_upd) ? cg.rr_upd[rhs] : 0.0;
+  const double* p = partial + (int64_t)rhs * bpr;
+  const int nt = (int)blockDim.x, t = (int)threadIdx.x;
+  double a[4] = {0.0, 0.0, 0.0, 0.0};
+  int k = t;
+  for (; k + 3 * nt < bpr; k += 4 * nt) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) a[i] += p[k + i * nt];
   }
-  if (threadIdx.x != 0) return;
-  const double v = red[0];
+  for (; k < bpr; k += nt) a[0] += p[k];
+  double s = wsum((a[0] + a[1]) + (a[2] + a[3]));
+  if ((t & 63) == 0) red[t >> 6] = s;
+  __syncthreads();
+  if (t != 0) return;
+  double v = red[0];
+  for (int w = 1; w < (nt >> 6); w++) v += red[w];
   if (out) out[rhs] = v;
   if (mode == RED_CG_ALPHA) {
     // d = <p, A p>  ->  a = rr / d
     cg.d[rhs] = v;
-    if (cg.alpha_prev) cg.alpha_prev[rhs] = cg.alpha[rhs];
-    if (cg.active[rhs]) {
-      cg.iters[rhs] += 1;
-      cg.rr_prev[rhs] = cg.rr[rhs];
+    if (cg.alpha_prev) cg.alpha_prev[rhs] = old_alpha;
+    if (was_active) {
+      cg.iters[rhs] = iters + 1;
+      cg.rr_prev[rhs] = old_rr;
       if (v == 0.0) {           // inv_cg.C:326-329
         cg.active[rhs] = 0;
         cg.status[rhs] = CG_STATUS_D_ZERO;
         cg.alpha[rhs] = 0.0;
       } else {
-        cg.alpha[rhs] = cg.rr[rhs] / v;
+        cg.alpha[rhs] = old_rr / v;
       }
     } else {
       cg.alpha[rhs] = 0.0;
     }
   } else if (mode == RED_CG_BETA) {
-    if (cg.active[rhs]) {
+    if (was_active) {
       cg.rr[rhs] = v;
-      if (cg.hist) cg.hist[(int64_t)rhs * cg.hist_len + (cg.iters[rhs] - 1) % cg.hist_len] = v;
-      if (v <= cg.stp[rhs]) {
+      if (cg.hist) cg.hist[(int64_t)rhs * cg.hist_len + (iters - 1) % cg.hist_len] = v;
+      if (v <= stp) {
         cg.active[rhs] = 0;
         cg.status[rhs] = CG_STATUS_CONVERGED;
         cg.beta[rhs] = 0.0;
-      } else if (cg.rr_upd && v < cg.delta2 * cg.rr_upd[rhs]) {
+      } else if (cg.rr_upd && v < cg.delta2 * rr_upd) {
         cg.active[rhs] = 0;
         cg.status[rhs] = CG_STATUS_NEED_UPDATE;
-        cg.beta[rhs] = v / cg.rr_prev[rhs];
-      } else if (cg.iters[rhs] >= cg.max_itr) {
+        cg.beta[rhs] = v / rr_prev;
+      } else if (iters >= cg.max_itr) {
         cg.active[rhs] = 0;
         cg.status[rhs] = CG_STATUS_MAXITER;
-        cg.beta[rhs] = v / cg.rr_prev[rhs];
+        cg.beta[rhs] = v / rr_prev;
       } else {
-        cg.beta[rhs] = v / cg.rr_prev[rhs];
+        cg.beta[rhs] = v / rr_prev;
       }
     }
   } else if (mode == RED_CG_INIT) {
     // initial |r|^2: decides whether any iteration runs (inv_cg.C:267-276)
     cg.rr[rhs] = v;
     cg.iters[rhs] = 0;
-    if (v <= cg.stp[rhs] || cg.max_itr <= 0) {
+    if (v <= stp || cg.max_itr <= 0) {
       cg.active[rhs] = 0;
       cg.status[rhs] = CG_STATUS_CONVERGED;
     } else {
@@ -555,9 +573,16 @@ hipError_t blas_axpy(int sx, const FieldRef& x, int sy, const FieldRef& y, const
   return hipErrorInvalidValue;
 }
 
+// threads of k_reduce_rhs: about four partials each, 64 to 1024
+static int reduce_threads(int bpr) {
+  int n = 64;
+  while (n < REDUCE_MAX && 4 * n < bpr) n <<= 1;
+  return n;
+}
+
 hipError_t reduce_rhs(const double* partial, int bpr, int nrhs, double* out, int mode, const CGScalars& cg,
                       hipStream_t s) {
-  hipLaunchKernelGGL(k_reduce_rhs, dim3(nrhs), dim3(256), 0, s, partial, bpr, out, mode, cg);
+  hipLaunchKernelGGL(k_reduce_rhs, dim3(nrhs), dim3(reduce_threads(bpr)), 0, s, partial, bpr, out, mode, cg);
   return hipGetLastError();
 }
 
