@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(256) k_xpay_x_t(FieldRef p, FieldRef r, FieldR
   const bool act = active[rhs] != 0;
   if (!act && a == 0.0) return;
   const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  using R = float;
+  using R = typename SpinTraits<SX>::R;
   cplx<typename SpinTraits<SP>::R> vp[12];
   spin_load<SP, typename SpinTraits<SP>::R>(p, e, vp);
   if (a != 0.0) {
@@ -372,7 +372,7 @@ __global__ void __launch_bounds__(256) k_cg_r_t(FieldRef r, FieldRef ap, const d
   ELEM_SETUP
   double n = 0;
   if (active[rhs]) {
-    using R = float;
+    using R = typename SpinTraits<SR>::R;
     const R a = R(alpha[rhs]);
     cplx<typename SpinTraits<SR>::R> vr[12];
     cplx<typename SpinTraits<SA>::R> va[12];
@@ -627,6 +627,7 @@ hipError_t blas_xpay_x_mixed(int sp, const FieldRef& p, int sr, const FieldRef& 
   CPSHIP_XPX(STORE_H, SpinH, STORE_H, SpinH, STORE_H, SpinH)
   CPSHIP_XPX(STORE_H, SpinH, STORE_H, SpinH, STORE_F, SpinF)
   CPSHIP_XPX(STORE_F, SpinF, STORE_F, SpinF, STORE_F, SpinF)
+  CPSHIP_XPX(STORE_D, SpinD, STORE_D, SpinD, STORE_D, SpinD)
 #undef CPSHIP_XPX
   return hipErrorInvalidValue;
 }
@@ -677,6 +678,7 @@ hipError_t blas_cg_r_mixed(int sr, const FieldRef& r, int sa, const FieldRef& ap
   if (sr == STORE_F && sa == STORE_H) hipLaunchKernelGGL((k_cg_r_t<SpinF, SpinH>), g, b, 0, s, r, ap, cg.alpha, cg.active, per_rhs, partial);
   else if (sr == STORE_H && sa == STORE_H) hipLaunchKernelGGL((k_cg_r_t<SpinH, SpinH>), g, b, 0, s, r, ap, cg.alpha, cg.active, per_rhs, partial);
   else if (sr == STORE_F && sa == STORE_F) hipLaunchKernelGGL((k_cg_r_t<SpinF, SpinF>), g, b, 0, s, r, ap, cg.alpha, cg.active, per_rhs, partial);
+  else if (sr == STORE_D && sa == STORE_D) hipLaunchKernelGGL((k_cg_r_t<SpinD, SpinD>), g, b, 0, s, r, ap, cg.alpha, cg.active, per_rhs, partial);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

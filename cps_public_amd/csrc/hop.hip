@@ -37,17 +37,25 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   if (P.m5post && (!std::is_same<SIN, SpinH>::value || P.kind != KIND_WILSON || P.nb != 16 || P.X.data || bs % 16))
     return hipErrorInvalidValue;
   if (P.rupd) {
-    // the CG residual update instead of the store (CLOV_NRR): half-precision
-    // DWF hops with X, element or spatial order, no variants
-    if (P.clov != CLOV_NONE || P.kind != KIND_DWF || !P.X.data || !P.R.data || !P.ralpha || !P.ractive || P.m5post ||
-        (P.flags & (HOP_SITEWAVE | HOP_LDS_LINKS | HOP_RHSGROUP | HOP_LINK_ROW)))
+    // the CG residual update instead of the store (CLOV_NRR), for the last hop
+    // of M^dag: half-precision or FP64 hops with X, element or spatial order;
+    // the FP64 Wilson kind also in the rhs-group mapping
+    constexpr bool D = std::is_same<SIN, SpinD>::value, H = std::is_same<SIN, SpinH>::value;
+    const bool group = (P.flags & HOP_RHSGROUP) != 0;
+    if (P.clov != CLOV_NONE || !P.dag || !P.X.data || !P.R.data || !P.ralpha || !P.ractive || P.m5post ||
+        (P.kind != KIND_DWF && !D) || (group && P.kind == KIND_DWF) ||
+        (P.flags & (HOP_SITEWAVE | HOP_LDS_LINKS | HOP_LINK_ROW)))
       return hipErrorInvalidValue;
-    if constexpr (std::is_same<SIN, SpinH>::value) {
-      if (P.dag) {
-        hipLaunchKernelGGL((k_hop<SIN, SOUT, LK, R, 1, KIND_DWF, false, CLOV_NRR, 0>), grid, block, 0, st, Q);
-      } else {
-        hipLaunchKernelGGL((k_hop<SIN, SOUT, LK, R, 0, KIND_DWF, false, CLOV_NRR, 0>), grid, block, 0, st, Q);
+    if constexpr (D || H) {
+#define CPSHIP_HOP_NRR(KIND, SW)                                                                             \
+  if (D && nt) hipLaunchKernelGGL((k_hop<SIN, SOUT, LK, R, 1, KIND, D, CLOV_NRR, SW>), grid, block, 0, st, Q); \
+  else hipLaunchKernelGGL((k_hop<SIN, SOUT, LK, R, 1, KIND, false, CLOV_NRR, SW>), grid, block, 0, st, Q);
+      if (P.kind == KIND_DWF) {
+        CPSHIP_HOP_NRR(KIND_DWF, 0)
+      } else if constexpr (D) {
+        if (group) { CPSHIP_HOP_NRR(KIND_WILSON, 3) } else { CPSHIP_HOP_NRR(KIND_WILSON, 0) }
       }
+#undef CPSHIP_HOP_NRR
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;

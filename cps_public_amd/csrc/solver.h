@@ -275,7 +275,8 @@ int clover_mdag_rupdate(Lattice& L, const cps_hip_op* op, int hprec, const Field
 // DWF M^dag of t3 with the CG residual step in the epilogue of its second
 // hop: r -= alpha[rhs] (M^dag t3) for the rhs with active[rhs], partial =
 // |r|^2 (FP16 r and hops; M^dag M p is never stored)
-int dwf_mdag_rupdate(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& r, const FieldRef& t3,
+bool mdag_rupdate_ok(const cps_hip_op* op, int hprec);
+int mdag_rupdate(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& r, const FieldRef& t3,
                      const FieldRef& t1, const double* alpha, const int* active, double* partial, int nrhs);
 int clover_build(Lattice& L, const double* kappas, int n_kappa, double csw);
 int clover_export(Lattice& L, int k, int cb, double* A);

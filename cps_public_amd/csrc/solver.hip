@@ -596,6 +596,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
       // order in every mapping, so a rhs-group choice that the count no
       // longer allows falls back to element order)
       for (const auto& kv : tune_cache) {
+        if (P.rupd) break;   // never timed: its rule is cheap and follows the count
         HopTuneKey k2 = kv.first;
         k2.nrhs = key.nrhs;
         if (k2 < key || key < k2) continue;
@@ -622,7 +623,25 @@ int tuned_launch(Lattice& L, HopParams& P) {
                     0.0};
     if (quad) best.flags = HOP_QUAD | (spatial_ok(L, P, def_block) ? HOP_SPATIAL : 0);
     // a launch that updates a field in place (rupd) is never timed on the
-    // live data: it keeps the fixed order of launches with partials
+    // live data: it keeps the fixed order of launches with partials.  One
+    // element per site: the rhs groups, which measured best wherever they
+    // divide the rhs (FP64 16^3x32 Wilson, 12 rhs: G = 4 146, 2 172, element
+    // order 245 us), and blocks of one wavefront where larger ones would leave
+    // CUs idle.  FP64 residuals that do not stay in the 256 MB cache between
+    // two kernels are stored around it.
+    if (P.rupd && P.prec == PREC_D_D18) {
+      if (P.nb == 1 && hop_chunk_partials(P)) {
+        if (per_rhs * P.nrhs < 256 * 256) best.block = 64;
+        for (int G : {4, 2}) {
+          const int f = HOP_RHSGROUP | ((G >> 2) << 6);
+          if (rhsgroup_ok(P, best.block, f)) {
+            best.flags = f;
+            break;
+          }
+        }
+      }
+      if (per_rhs * P.nrhs * 192 > (int64_t(32) << 20)) best.flags |= HOP_NT_STORE;
+    }
     if (tuning_enabled() && !P.rupd) {
       std::vector<int> blocks;
       if (P.partial && !hop_chunk_partials(P)) blocks.push_back(def_block);
@@ -731,11 +750,17 @@ int apply_m(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& out, co
   return hop(L, op, hprec, out, t, 1, dag, -k * k, in, 1.0, partial, nrhs);
 }
 
-// M^dag t3 = t3 - kappa^2 D^dag D^dag t3 (dwf_mdag.C:32-62) with r -= alpha
-// M^dag t3 and |r|^2 in the epilogue of the second hop (CLOV_NRR)
-int dwf_mdag_rupdate(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& r, const FieldRef& t3,
-                     const FieldRef& t1, const double* alpha, const int* active, double* partial, int nrhs) {
-  if (op->kind != CPS_HIP_OP_DWF || hprec == PREC_D_D18 || hprec == PREC_F_F12) return CPS_HIP_ERR_ARG;
+// M^dag t3 = t3 - kappa^2 D^dag D^dag t3 (wilson_m.C:73-91, dwf_mdag.C:32-62)
+// with r -= alpha M^dag t3 and |r|^2 in the epilogue of the second hop
+// (CLOV_NRR): DWF in half precision and FP64, Wilson in FP64
+bool mdag_rupdate_ok(const cps_hip_op* op, int hprec) {
+  if (op->kind == CPS_HIP_OP_WILSON) return hprec == PREC_D_D18;
+  return op->kind == CPS_HIP_OP_DWF && hprec != PREC_F_F12;
+}
+
+int mdag_rupdate(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& r, const FieldRef& t3,
+                 const FieldRef& t1, const double* alpha, const int* active, double* partial, int nrhs) {
+  if (!mdag_rupdate_ok(op, hprec)) return CPS_HIP_ERR_ARG;
   const double k = op_kappa(op);
   int rc = hop(L, op, hprec, t1, t3, 0, 1, 1.0, null_field(), 0.0, nullptr, nrhs);
   if (rc) return rc;
@@ -1000,6 +1025,14 @@ int cg_double_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int
   CGState cg;
   rc = cg.alloc(L, nrhs, 0);
   if (rc) return rc;
+  // Of the 10 passes over a vector that the CG step makes beside the operator
+  // (x, r, p and A p), 3 are saved: x += alpha p waits for the kernel that
+  // reads p next, p = r + beta p, and r -= alpha A p runs in the epilogue of
+  // the operator's last hop, so that A p is never stored
+  // (CPS_HIP_LAGGED_X=0, CPS_HIP_R_IN_HOP=0: separate passes)
+  const cps_hip_tuning tn = tuning();
+  const bool lagged = tn.lagged_x != 0;
+  const bool r_in_hop = lagged && tn.r_in_hop != 0 && mdag_rupdate_ok(op, PREC_D_D18);
   cg.s.max_itr = arg->max_num_iter - 1;
   {
     std::vector<double> rsd(nrhs, arg->stop_rsd);
@@ -1029,9 +1062,26 @@ int cg_double_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int
   Progress prog("fp64");
   IterGraph iter_graph(arg->use_graph != 0);
   RhsWindow win(L, nrhs);
+  const std::vector<double> zeros(nrhs, 0.0);
+  if (lagged) {   // the first direction is r; no step of x is pending
+    CPSHIP_CHECK(hipMemcpyAsync(cg.s.alpha, zeros.data(), nrhs * sizeof(double), hipMemcpyHostToDevice, L.stream));
+    CPSHIP_CHECK(hipMemcpyAsync(cg.s.beta, zeros.data(), nrhs * sizeof(double), hipMemcpyHostToDevice, L.stream));
+  }
+  // the pending steps x += alpha p of rhs lo .. lo+n-1
+  auto flush_x = [&](int lo, int m) -> int {
+    if (!lagged) return 0;
+    CPSHIP_CHECK(blas_axpy(STORE_D, rhs_view(p.ref(), o.per_rhs, lo), STORE_D, rhs_view(x.ref(), o.per_rhs, lo),
+                           cg.s.alpha + lo, 0.0, o.per_rhs, m, bsb, L.stream));
+    CPSHIP_CHECK(hipMemcpyAsync(cg.s.alpha + lo, zeros.data(), m * sizeof(double), hipMemcpyHostToDevice, L.stream));
+    return 0;
+  };
   while (any_active() && done_iters < max_itr) {
     prog.tick(L, done_iters, act, cg.s.rr);
-    if (win.update(act)) iter_graph.reset();
+    const int old_lo = win.lo, old_n = win.n();
+    if (win.update(act)) {
+      if ((rc = flush_x(old_lo, old_n))) return rc;
+      iter_graph.reset();
+    }
     const int nw = win.n();
     const FieldRef xw = rhs_view(x.ref(), o.per_rhs, win.lo), pw = rhs_view(p.ref(), o.per_rhs, win.lo);
     const FieldRef rw = rhs_view(r.ref(), o.per_rhs, win.lo), apw = rhs_view(ap.ref(), o.per_rhs, win.lo);
@@ -1039,12 +1089,28 @@ int cg_double_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int
     const int todo = std::min(chunk, max_itr - done_iters);
     rc = iter_graph.run(L, todo, [&]() -> int {
       // mmp = MdagM p, d = |M p|^2 (inv_cg.C:302)
-      int e = apply_mdagm(L, op, PREC_D_D18, apw, pw, t1.ref(), t2.ref(), part, nw);
+      int e;
+      if (lagged)
+        CPSHIP_CHECK(blas_xpay_x_mixed(STORE_D, pw, STORE_D, rw, STORE_D, xw, sw.alpha, sw.beta, sw.active, o.per_rhs,
+                                       nw, bsb, L.stream));
+      if (r_in_hop) {
+        e = apply_m(L, op, PREC_D_D18, t2.ref(), pw, t1.ref(), 0, part, nw);
+        if (e) return e;
+        CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_ALPHA, sw, L.stream));
+        e = mdag_rupdate(L, op, PREC_D_D18, rw, t2.ref(), t1.ref(), sw.alpha, sw.active, part, nw);
+        if (e) return e;
+        CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_BETA, sw, L.stream));
+        return 0;
+      }
+      e = apply_mdagm(L, op, PREC_D_D18, apw, pw, t1.ref(), t2.ref(), part, nw);
       if (e) return e;
       CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_ALPHA, sw, L.stream));
-      CPSHIP_CHECK(blas_cg_xr_d(xw, pw, rw, apw, sw, o.per_rhs, nw, bsb, part, L.stream));
+      if (lagged)
+        CPSHIP_CHECK(blas_cg_r_mixed(STORE_D, rw, STORE_D, apw, sw, o.per_rhs, nw, bsb, part, L.stream));
+      else
+        CPSHIP_CHECK(blas_cg_xr_d(xw, pw, rw, apw, sw, o.per_rhs, nw, bsb, part, L.stream));
       CPSHIP_CHECK(reduce_rhs(part, bpr_blas, nw, nullptr, RED_CG_BETA, sw, L.stream));
-      CPSHIP_CHECK(blas_xpay(STORE_D, pw, rw, sw.beta, sw.active, o.per_rhs, nw, bsb, L.stream));
+      if (!lagged) CPSHIP_CHECK(blas_xpay(STORE_D, pw, rw, sw.beta, sw.active, o.per_rhs, nw, bsb, L.stream));
       return 0;
     });
     if (rc) return rc;
@@ -1052,6 +1118,7 @@ int cg_double_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int
     rc = sync_read(L, act.data(), cg.s.active, nrhs * sizeof(int));
     if (rc) return rc;
   }
+  if ((rc = flush_x(win.lo, win.n()))) return rc;
   win.lo = 0;
   win.hi = nrhs;
   L.win_lo = 0;
@@ -1345,7 +1412,7 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
         int e = apply_m(L, op, hprec, t3s.ref(), pw, t1s.ref(), 0, part, nw);
         if (e) return e;
         CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_ALPHA, sw, L.stream));
-        e = dwf_mdag_rupdate(L, op, hprec, rsw, t3s.ref(), t1s.ref(), sw.alpha, sw.active, part, nw);
+        e = mdag_rupdate(L, op, hprec, rsw, t3s.ref(), t1s.ref(), sw.alpha, sw.active, part, nw);
         if (e) return e;
         CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_BETA, sw, L.stream));
         return 0;
