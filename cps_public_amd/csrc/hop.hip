@@ -19,7 +19,9 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   // partials per 64-site chunk: wavefront-aligned blocks, and a mapping that
   // keeps a chunk's sites in one block (element order or the rhs groups)
   Q.chunk_part = hop_chunk_partials(P) ? 1 : 0;
-  if (Q.chunk_part && (bs % 64 || (P.flags & (HOP_SPATIAL | HOP_SITEWAVE)))) return hipErrorInvalidValue;
+  if (Q.chunk_part && (bs % 64 || (P.flags & HOP_SITEWAVE) ||
+                       ((P.flags & HOP_SPATIAL) && !(P.flags & HOP_RHSGROUP))))
+    return hipErrorInvalidValue;
   const bool nt = (P.flags & HOP_NT_STORE) != 0;
   // HOP_LDS_LINKS: half-precision spinors, one link per thread to stage
   const bool lds = (P.flags & HOP_LDS_LINKS) != 0;

@@ -493,7 +493,7 @@ __device__ __forceinline__ void chunk_partial_elem(const HopParams& P, int rhs, 
 // over the S lanes of each rhs gives the first log2 S levels of that tree;
 // the G wavefronts of a chunk (in one block, G <= W) then combine pairwise,
 // (a0 + a1) + (a2 + a3), as the remaining levels.
-__device__ __forceinline__ void chunk_partial_rhsgroup(const HopParams& P, int64_t sb64, double v) {
+__device__ __forceinline__ void chunk_partial_rhsgroup(const HopParams& P, int rhs, int64_t pslot, double v) {
   __shared__ double cred[16];
   const int s_shift = 6 - P.rg_shift, S = 1 << s_shift, G = 1 << P.rg_shift;
   for (int m = 1; m < S; m <<= 1) v += __shfl_xor(v, m);
@@ -506,11 +506,7 @@ __device__ __forceinline__ void chunk_partial_rhsgroup(const HopParams& P, int64
     // G is 2 or 4 (G <= W <= 4)
     const double* cw = cred + c * G * G + g;
     const double sum = G == 2 ? cw[0] + cw[G] : (cw[0] + cw[G]) + (cw[2 * G] + cw[3 * G]);
-    const int sb = (int)sb64;
-    const int per_g = P.nsites_out / (W << s_shift);
-    const int rg = sb / per_g, sblk = sb - rg * per_g;
-    const int64_t rhs = ((int64_t)rg << P.rg_shift) + g;
-    P.partial[rhs * (P.nsites_out >> 6) + (int64_t)sblk * (W >> P.rg_shift) + c] = sum;
+    P.partial[(int64_t)((rhs & ~(G - 1)) + g) * (P.nsites_out >> 6) + pslot + c] = sum;
   }
 }
 
@@ -608,20 +604,37 @@ __device__ __forceinline__ void hop_block_sites(const HopParams& P, int el0, int
 // HOP_RHSGROUP decode (Wilson kind, nb a power of two, no partials): lane =
 // (g S + q) nb + j with g < G rhs and q < S = 64 / (G nb) consecutive sites;
 // logical block sb = (rhs group, block of W S sites), W wavefronts per block
-__device__ __forceinline__ HopElem hop_decode_rhsgroup(const HopParams& P, int64_t sb64) {
+__device__ __forceinline__ HopElem hop_decode_rhsgroup(const HopParams& P, int64_t sb64, int64_t nsub64) {
   HopElem E;
   const int sb = (int)sb64;
   const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6), W = (int)(blockDim.x >> 6);
   const int s_shift = 6 - P.rg_shift - P.nb_shift;   // log2 S
-  const int per_g = P.nsites_out / (W << s_shift);
-  const int rg = sb / per_g;
-  const int sblk = sb - rg * per_g;
+  int rg, sblk, b = 0;
+  if (P.flags & HOP_SPATIAL) {
+    // sb = (spatial block b = XCD, tile of rhs groups, site block, group of
+    // the tile): the groups of a tile run over the same sites together
+    const int per_b = (int)nsub64 >> 3;
+    b = sb / per_b;
+    const int n_in = sb - b * per_b;
+    const int spb = P.perm_S / (W << s_shift), ng = P.nrhs >> P.rg_shift;
+    const int tile = n_in / (spb * P.rg_tile), rem = n_in - tile * (spb * P.rg_tile);
+    const int left = ng - tile * P.rg_tile, cnt = left < P.rg_tile ? left : P.rg_tile;
+    sblk = rem / cnt;
+    rg = tile * P.rg_tile + rem - sblk * cnt;
+  } else {
+    const int per_g = P.nsites_out / (W << s_shift);
+    rg = sb / per_g;
+    sblk = sb - rg * per_g;
+  }
   const int gq = lane >> P.nb_shift;
   const int g = gq >> s_shift;
   E.j = lane & (P.nb - 1);
   E.rhs = (rg << P.rg_shift) + g;
-  E.site = ((sblk * W + w) << s_shift) + (gq - (g << s_shift));
-  E.pslot = 0;   // no partials in this mode
+  const int q = ((sblk * W + w) << s_shift) + (gq - (g << s_shift));
+  E.site = (P.flags & HOP_SPATIAL) ? (int)P.perm[(int64_t)b * P.perm_S + q] : q;
+  // partials (one element per site): the block's first chunk of 64 sites in
+  // the order of the sweep
+  E.pslot = ((int64_t)b * P.perm_S + ((int64_t)(sblk * W) << s_shift)) >> 6;
   E.qb = E.nsl = E.sl = E.b = 0;
   return E;
 }
@@ -1152,13 +1165,13 @@ __global__ void __launch_bounds__(256, HopWaves<SIN>::value) k_hop(HopParams P) 
   const int64_t nsub = (int64_t)gridDim.x;
   const int64_t hb = logical_block(blockIdx.x, gridDim.x, !(P.flags & HOP_NO_XCD_REMAP));
   const HopElem E = SW == 1 ? hop_decode_sitewave(P, hb, nsub)
-                   : SW == 3 ? hop_decode_rhsgroup(P, hb) : hop_decode<KIND>(P, hb, nsub);
+                   : SW == 3 ? hop_decode_rhsgroup(P, hb, nsub) : hop_decode<KIND>(P, hb, nsub);
   const Nbr N = hop_nbr<KIND>(P, E);
   const double nrm = hop_element<SIN, SOUT, LK, R, DAG, KIND, NT, CLOV, SW == 2, SW == 4>(
       P, E, N, reinterpret_cast<uint32_t*>(hop_lds_area));
   if (P.partial) {
     if (!P.chunk_part) block_partial<double>(nrm, P.partial, E.pslot);
-    else if constexpr (SW == 3) chunk_partial_rhsgroup(P, hb, nrm);
+    else if constexpr (SW == 3) chunk_partial_rhsgroup(P, E.rhs, E.pslot, nrm);
     else chunk_partial_elem(P, E.rhs, E.site, nrm);
   }
 }

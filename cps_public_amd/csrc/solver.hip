@@ -569,8 +569,6 @@ int tuned_launch(Lattice& L, HopParams& P) {
     CPSHIP_CHECK(launch_hop(P, L.stream));
     return 0;
   }
-  if (L.perm_state >= 0 && L.g.Vcb % 8 == 0 && L.ensure_perm() == 0)
-    P.perm = (const uint32_t*)(P.kind == KIND_DWF ? L.perm5.p : L.perm.p);
   if (P.clov == CLOV_KS) {
     // a mass per rhs: one kernel in element order (no variants to time)
     P.block = def_block;
@@ -588,27 +586,34 @@ int tuned_launch(Lattice& L, HopParams& P) {
     if (f != tune_cache.end()) {
       chosen = f->second;
       have = true;
-    } else {
-      // the same shape tuned for another rhs count (a CG's active-rhs window
-      // shrinking): reuse that choice where it is valid for this count (for
-      // launches with per-block partials it is the fixed-order choice, which
-      // does not depend on the count; chunk partials are summed in the same
-      // order in every mapping, so a rhs-group choice that the count no
-      // longer allows falls back to element order)
-      for (const auto& kv : tune_cache) {
-        if (P.rupd) break;   // never timed: its rule is cheap and follows the count
-        HopTuneKey k2 = kv.first;
-        k2.nrhs = key.nrhs;
-        if (k2 < key || key < k2) continue;
-        chosen = kv.second;
-        if ((chosen.flags & HOP_SITEWAVE) && !sitewave_ok(L, P, chosen.block, (chosen.flags & HOP_SPATIAL) != 0))
-          chosen.flags &= ~HOP_SITEWAVE;
-        if ((chosen.flags & HOP_RHSGROUP) && !rhsgroup_ok(P, chosen.block, chosen.flags))
-          chosen.flags &= ~(HOP_RHSGROUP | (3 << 6));
-        have = true;
-        tune_cache.emplace(key, chosen);
-        break;
+    }
+  }
+  // the spatial order's table, built on the handle's first use of it
+  if ((!have || (chosen.flags & HOP_SPATIAL)) && L.perm_state >= 0 && L.g.Vcb % 8 == 0 && L.ensure_perm() == 0)
+    P.perm = (const uint32_t*)(P.kind == KIND_DWF ? L.perm5.p : L.perm.p);
+  if (!have) {
+    std::lock_guard<std::mutex> lk(tune_mu);
+    // the same shape tuned for another rhs count (a CG's active-rhs window
+    // shrinking): reuse that choice where it is valid for this count (for
+    // launches with per-block partials it is the fixed-order choice, which
+    // does not depend on the count; chunk partials are summed in the same
+    // order in every mapping, so a rhs-group choice that the count no
+    // longer allows falls back to element order)
+    for (const auto& kv : tune_cache) {
+      if (P.rupd) break;   // never timed: its rule is cheap and follows the count
+      HopTuneKey k2 = kv.first;
+      k2.nrhs = key.nrhs;
+      if (k2 < key || key < k2) continue;
+      chosen = kv.second;
+      if ((chosen.flags & HOP_SITEWAVE) && !sitewave_ok(L, P, chosen.block, (chosen.flags & HOP_SPATIAL) != 0))
+        chosen.flags &= ~HOP_SITEWAVE;
+      if ((chosen.flags & HOP_RHSGROUP) && !rhsgroup_ok(P, chosen.block, chosen.flags)) {
+        chosen.flags &= ~(HOP_RHSGROUP | (3 << 6));
+        if ((chosen.flags & HOP_SPATIAL) && !spatial_ok(L, P, chosen.block)) chosen.flags &= ~HOP_SPATIAL;
       }
+      have = true;
+      tune_cache.emplace(key, chosen);
+      break;
     }
   }
   if (!have) {
@@ -661,7 +666,10 @@ int tuned_launch(Lattice& L, HopParams& P) {
         cand = {HOP_QUAD, HOP_QUAD | HOP_NO_XCD_REMAP, HOP_QUAD | HOP_SPATIAL};
       for (int f = 0; f < 32 && !quad; f++) cand.push_back(f);
       for (int g = 0; g < 4 && !quad; g++)
-        for (int nt = 0; nt < 2; nt++) cand.push_back(HOP_RHSGROUP | (g << 6) | nt);
+        for (int nt = 0; nt < 2; nt++) {
+          cand.push_back(HOP_RHSGROUP | (g << 6) | nt);
+          cand.push_back(HOP_RHSGROUP | (g << 6) | HOP_SPATIAL | nt);
+        }
       for (int f = 0; f < 8 && !quad; f++) cand.push_back(HOP_LINK_ROW | f);
       for (int b : blocks)
         for (int f : cand) {
@@ -687,7 +695,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
             continue;   // CPS_HIP_HOP_MODE=rhsgroup
           }
           if (f & HOP_SPATIAL) {
-            if ((f & HOP_NO_XCD_REMAP) || !spatial_ok(L, P, b)) continue;
+            if ((f & HOP_NO_XCD_REMAP) || (!(f & HOP_RHSGROUP) && !spatial_ok(L, P, b))) continue;
           }
           if ((f & HOP_SITEWAVE) && !sitewave_ok(L, P, b, (f & HOP_SPATIAL) != 0)) continue;
           if ((f & HOP_LDS_LINKS) && ((f & HOP_SITEWAVE) || !lds_links_ok(P, b))) continue;
