@@ -141,7 +141,7 @@ int Lattice::import_gauge_canonical(const double* u_canon) {
   int rc = io.ensure(n * sizeof(double));
   if (rc) return rc;
   if ((rc = io2.ensure(n * sizeof(double)))) return rc;
-  CPSHIP_CHECK(hipMemcpyAsync(io.p, u_canon, n * sizeof(double), hipMemcpyHostToDevice, stream));
+  CPSHIP_CHECK(stager.to_device(io.p, u_canon, n * sizeof(double), stream));
   const int64_t nt = (int64_t)8 * g.Vcb;
   hipLaunchKernelGGL(k_gauge_canon_to_wilson, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, stream,
                      (const double*)io.p, (double*)io2.p, g);
@@ -181,16 +181,15 @@ int cps_hip_fmatinv(cps_hip_lattice* lat, const cps_hip_op* op, double* out, con
   const bool mob = op->kind == CPS_HIP_OP_MOBIUS;
   // the Moebius CG solves the 2 kappa_b-normalised system
   const double g = mob ? op->mobius_b * (4 - op->m5) + op->a5_inv : 1.0;
-  CPSHIP_CHECK(hipMemcpyAsync(L.io.p, in, bytes, hipMemcpyHostToDevice, L.stream));
-  CPSHIP_CHECK(hipMemcpyAsync(L.io2.p, out, bytes, hipMemcpyHostToDevice, L.stream));
+  CPSHIP_CHECK(L.stager.to_device(L.io.p, in, bytes, L.stream));
+  CPSHIP_CHECK(L.stager.to_device(L.io2.p, out, bytes, L.stream));
   if ((rc = pack_canonical(L, op->kind, (const double*)L.io.p, fo, fe, nrhs, 1.0))) return rc;
   // the initial guess: its odd half starts the CG (the even half is rebuilt)
   if ((rc = pack_canonical(L, op->kind, (const double*)L.io2.p, x, eo, nrhs, g))) return rc;
   if (mob && (rc = mobius_dminus_fields(L, op, fo, fe, nrhs))) return rc;
   if ((rc = matinv_device(L, op, fo, fe, x, eo, nrhs, arg, res))) return rc;
   if ((rc = unpack_canonical(L, op->kind, x, eo, (double*)L.io2.p, nrhs, 1.0 / g))) return rc;
-  CPSHIP_CHECK(hipMemcpyAsync(out, L.io2.p, bytes, hipMemcpyDeviceToHost, L.stream));
-  CPSHIP_CHECK(hipStreamSynchronize(L.stream));
+  CPSHIP_CHECK(L.stager.to_host(out, L.io2.p, bytes, L.stream));
   return 0;
 }
 

@@ -1,0 +1,129 @@
+// Staged copies of large pageable host vectors.
+//
+// A pageable hipMemcpyAsync moves the data through the runtime's own staging
+// buffer with one host thread: 12-15 GB/s, and a vector that the caller has
+// just allocated is page-faulted in by that thread as well.  Here up to 8
+// threads copy 2 MiB chunks to and from pinned buffers (two each, so a
+// thread's host copy runs beside the DMA of its other buffer).
+//
+// Domain-wall M^dag M of 16^3x32, Ls 16, on host vectors (201 MB each way, a
+// fresh output array): 27.5 -> 12.4 ms; a 12-source Wilson propagator (302 MB
+// out) 168 -> 145 ms.
+#include "hostcopy.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <thread>
+#include <vector>
+
+namespace cpship {
+
+HostStager::~HostStager() {
+  for (hipEvent_t e : done)
+    if (e) (void)hipEventDestroy(e);
+  if (pinned) (void)hipHostFree(pinned);
+}
+
+bool HostStager::ready() {
+  if (pinned) return true;
+  for (hipEvent_t& e : done)
+    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      e = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+  void* p = nullptr;
+  if (hipHostMalloc(&p, WORKERS * BUFS * CHUNK, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  pinned = static_cast<char*>(p);
+  return true;
+}
+
+// Every chunk is taken by one worker; a worker's failure stops the others and
+// is returned.
+hipError_t HostStager::run(char* dev, char* host, size_t bytes, hipStream_t st, bool up) {
+  const size_t nchunk = (bytes + CHUNK - 1) / CHUNK;
+  int device = 0;
+  hipError_t rc = hipGetDevice(&device);
+  if (rc != hipSuccess) return rc;
+  std::atomic<size_t> next{0};
+  std::atomic<int> failed{(int)hipSuccess};
+  auto work = [&](int w) {
+    auto check = [&](hipError_t e) {
+      if (e != hipSuccess) failed.store((int)e);
+      return e == hipSuccess;
+    };
+    if (!check(hipSetDevice(device))) return;
+    char* buf[BUFS];
+    hipEvent_t ev[BUFS];
+    size_t at[BUFS], len[BUFS] = {};   // chunk in flight in each buffer (len 0: none)
+    for (int b = 0; b < BUFS; b++) {
+      buf[b] = pinned + (size_t)(w * BUFS + b) * CHUNK;
+      ev[b] = done[w * BUFS + b];
+    }
+    auto settle = [&](int b) {
+      if (!len[b]) return true;
+      const bool ok = check(hipEventSynchronize(ev[b]));
+      if (ok && !up) std::memcpy(host + at[b], buf[b], len[b]);
+      len[b] = 0;
+      return ok;
+    };
+    int b = 0;
+    for (;; b = (b + 1) % BUFS) {
+      if (!settle(b) || failed.load() != (int)hipSuccess) break;
+      const size_t c = next.fetch_add(1);
+      if (c >= nchunk) break;
+      const size_t off = c * CHUNK, n = std::min(CHUNK, bytes - off);
+      if (up) std::memcpy(buf[b], host + off, n);
+      if (!check(up ? hipMemcpyAsync(dev + off, buf[b], n, hipMemcpyHostToDevice, st)
+                    : hipMemcpyAsync(buf[b], dev + off, n, hipMemcpyDeviceToHost, st)) ||
+          !check(hipEventRecord(ev[b], st)))
+        break;
+      at[b] = off;
+      len[b] = n;
+    }
+    // the buffers are free again when the call returns, also after a failure
+    for (int k = 0; k < BUFS; k++) settle((b + k) % BUFS);
+  };
+  const int workers = (int)std::min<size_t>({(size_t)WORKERS, nchunk, std::max(1u, std::thread::hardware_concurrency())});
+  std::vector<std::thread> pool;
+  try {
+    pool.reserve(workers - 1);
+    for (int w = 1; w < workers; w++) pool.emplace_back(work, w);
+  } catch (...) {   // fewer threads: the others take their chunks
+  }
+  work(0);
+  for (std::thread& t : pool) t.join();
+  return (hipError_t)failed.load();
+}
+
+// Vectors below 8 chunks, and host memory that the runtime knows (pinned, so
+// that the DMA reads it directly), take a plain copy.
+static bool worth_staging(const void* host, size_t bytes) {
+  if (bytes < 8 * HostStager::CHUNK) return false;
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return a.type == hipMemoryTypeUnregistered;
+}
+
+hipError_t HostStager::to_device(void* dev, const void* host, size_t bytes, hipStream_t st) {
+  if (!worth_staging(host, bytes) || !ready()) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+  return run(static_cast<char*>(dev), const_cast<char*>(static_cast<const char*>(host)), bytes, st, true);
+}
+
+hipError_t HostStager::to_host(void* host, const void* dev, size_t bytes, hipStream_t st) {
+  hipError_t rc;
+  if (!worth_staging(host, bytes) || !ready())
+    rc = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
+  else
+    rc = run(const_cast<char*>(static_cast<const char*>(dev)), static_cast<char*>(host), bytes, st, false);
+  return rc == hipSuccess ? hipStreamSynchronize(st) : rc;
+}
+
+}  // namespace cpship

@@ -218,7 +218,6 @@ extern "C" int cps_hip_qpropw_point(cps_hip_lattice* lat, const cps_hip_op* op, 
   } else {
     CPSHIP_CHECK(launch_gather<CPS_HIP_OP_WILSON>(x, eo, L.g, o.per_rhs, L.ls, fac, pd, L.stream));
   }
-  CPSHIP_CHECK(hipMemcpyAsync(prop, L.io.p, pbytes, hipMemcpyDeviceToHost, L.stream));
-  CPSHIP_CHECK(hipStreamSynchronize(L.stream));
+  CPSHIP_CHECK(L.stager.to_host(prop, L.io.p, pbytes, L.stream));
   return 0;
 }

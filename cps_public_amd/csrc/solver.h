@@ -7,6 +7,7 @@
 #include "blas.h"
 #include "cps_hip_internal.h"
 #include "hop.h"
+#include "hostcopy.h"
 #include "layout.h"
 
 namespace cpship {
@@ -84,6 +85,7 @@ struct Lattice {
   int set_hop_phase(HopParams& P, int hprec) const;
   std::vector<Field> scratch;
   DevBuf partial, scal, io, io2;
+  HostStager stager;   // large copies from and to the caller's host vectors
   DevBuf nbr, nbr_neg;   // neighbour table of the geometry (hop kernels)
   // spatial site order of the HOP_SPATIAL launches (built on first use),
   // perm for one parity and perm5 for both (DWF fields): 0 not built, 1

@@ -841,7 +841,7 @@ int upload(Lattice& L, const double* host, Field& f, const OpLayout& o, int cb5,
     DevBuf& io = slot_io ? L.io2 : L.io;
     int rc = io.ensure((size_t)n * 24 * sizeof(double));
     if (rc) return rc;
-    CPSHIP_CHECK(hipMemcpyAsync(io.p, host, (size_t)n * 24 * sizeof(double), hipMemcpyHostToDevice, L.stream));
+    CPSHIP_CHECK(L.stager.to_device(io.p, host, (size_t)n * 24 * sizeof(double), L.stream));
     src = (const double*)io.p;
   }
   CPSHIP_CHECK(pack_spinor(f.storage, src, f.ref(), o.map, L.g.Vcb, L.ls, cb5, n, L.stream));
@@ -858,8 +858,7 @@ int download(Lattice& L, const Field& f, double* host, const OpLayout& o, int cb
   int rc = L.io.ensure((size_t)n * 24 * sizeof(double));
   if (rc) return rc;
   CPSHIP_CHECK(unpack_spinor(f.storage, f.ref(), (double*)L.io.p, o.map, L.g.Vcb, L.ls, cb5, n, L.stream));
-  CPSHIP_CHECK(hipMemcpyAsync(host, L.io.p, (size_t)n * 24 * sizeof(double), hipMemcpyDeviceToHost, L.stream));
-  CPSHIP_CHECK(hipStreamSynchronize(L.stream));
+  CPSHIP_CHECK(L.stager.to_host(host, L.io.p, (size_t)n * 24 * sizeof(double), L.stream));
   return 0;
 }
 
