@@ -34,11 +34,20 @@ __device__ __forceinline__ void block_partial_d(double v, double* partial, int64
   }
 }
 
-// grid: (blocks_per_rhs, nrhs); element e = rhs*per_rhs + blockIdx.x*blockDim.x + tid
-#define ELEM_SETUP                                                        \
-  const int rhs = blockIdx.y;                                             \
-  const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; \
+// grid: (blocks_per_rhs, nrhs); element e = rhs*per_rhs + i, i = blockIdx.x*blockDim.x + tid.  Threads past the
+// rhs's last element (in its last block) read element 0 and neither store nor count.
+#define ELEM_SETUP                                                                   \
+  const int rhs = blockIdx.y;                                                        \
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;                  \
+  const bool in = i < per_rhs;                                                       \
+  const int64_t e = (int64_t)rhs * per_rhs + (in ? i : 0);                           \
   const int64_t slot = (int64_t)rhs * gridDim.x + blockIdx.x;
+
+// kernels without a reduction leave such threads
+#define ELEM_OR_RETURN                                                               \
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;                  \
+  if (i >= per_rhs) return;                                                          \
+  const int64_t e = (int64_t)blockIdx.y * per_rhs + i;
 
 template <typename S>
 __global__ void __launch_bounds__(256) k_norm(FieldRef x, int64_t per_rhs, double* partial) {
@@ -49,7 +58,7 @@ __global__ void __launch_bounds__(256) k_norm(FieldRef x, int64_t per_rhs, doubl
   double n = 0;
 #pragma unroll
   for (int c = 0; c < 12; c++) n += double(v[c].re) * v[c].re + double(v[c].im) * v[c].im;
-  block_partial_d(n, partial, slot);
+  block_partial_d(in ? n : 0.0, partial, slot);
 }
 
 template <typename S>
@@ -62,7 +71,7 @@ __global__ void __launch_bounds__(256) k_redot(FieldRef x, FieldRef y, int64_t p
   double n = 0;
 #pragma unroll
   for (int c = 0; c < 12; c++) n += double(a[c].re) * b[c].re + double(a[c].im) * b[c].im;
-  block_partial_d(n, partial, slot);
+  block_partial_d(in ? n : 0.0, partial, slot);
 }
 
 // Re <x, y> with x and y in different storages
@@ -78,7 +87,7 @@ __global__ void __launch_bounds__(256) k_redot_t(FieldRef x, FieldRef y, int64_t
   double n = 0;
 #pragma unroll
   for (int c = 0; c < 12; c++) n += double(a[c].re) * double(b[c].re) + double(a[c].im) * double(b[c].im);
-  block_partial_d(n, partial, slot);
+  block_partial_d(in ? n : 0.0, partial, slot);
 }
 
 // r = b - a (FP64), optional |r|^2
@@ -93,8 +102,8 @@ __global__ void __launch_bounds__(256) k_sub_norm_d(FieldRef b, FieldRef a, Fiel
     va[c] = cmk<double>(vb[c].re - va[c].re, vb[c].im - va[c].im);
     n += va[c].re * va[c].re + va[c].im * va[c].im;
   }
-  spin_store<SpinD, double>(r, e, va);
-  if (partial) block_partial_d(n, partial, slot);
+  if (in) spin_store<SpinD, double>(r, e, va);
+  if (partial) block_partial_d(in ? n : 0.0, partial, slot);
 }
 
 // x += a p ; r -= a Ap ; |r|^2   (inv_cg.C:340-349), skipped for inactive rhs
@@ -103,7 +112,7 @@ __global__ void __launch_bounds__(256) k_cg_xr_d(FieldRef x, FieldRef p, FieldRe
                                                 double* partial) {
   ELEM_SETUP
   double n = 0;
-  if (active[rhs]) {
+  if (in && active[rhs]) {
     const double a = alpha[rhs];
     {   // x += a p
       cplx<double> vx[12], vp[12];
@@ -125,7 +134,7 @@ __global__ void __launch_bounds__(256) k_cg_xr_d(FieldRef x, FieldRef p, FieldRe
       spin_store<SpinD, double>(r, e, vr);
     }
   }
-  block_partial_d(n, partial, slot);
+  block_partial_d(in ? n : 0.0, partial, slot);
 }
 
 // p = b p + r for active rhs (inv_cg.C:360)
@@ -133,7 +142,7 @@ template <typename S>
 __global__ void __launch_bounds__(256) k_xpay(FieldRef p, FieldRef r, const double* beta, const int* active, int64_t per_rhs) {
   const int rhs = blockIdx.y;
   if (!active[rhs]) return;
-  const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  ELEM_OR_RETURN
   using R = typename SpinTraits<S>::R;
   const R b = R(beta[rhs]);
   cplx<R> vp[12], vr[12];
@@ -149,7 +158,7 @@ template <typename SX, typename SY>
 __global__ void __launch_bounds__(256) k_axpy(FieldRef x, FieldRef y, const double* a, double a_const, int64_t per_rhs) {
   const int rhs = blockIdx.y;
   if (a && a[rhs] == 0.0) return;   // a per-rhs coefficient of 0 leaves y as it is
-  const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  ELEM_OR_RETURN
   using RX = typename SpinTraits<SX>::R;
   using RY = typename SpinTraits<SY>::R;
   const RY c = RY(a ? a[rhs] : a_const);
@@ -169,7 +178,7 @@ __global__ void __launch_bounds__(256) k_cg_xr_t(FieldRef x, FieldRef p, FieldRe
                           const int* active, int64_t per_rhs, double* partial) {
   ELEM_SETUP
   double n = 0;
-  if (active[rhs]) {
+  if (in && active[rhs]) {
     using R = float;
     const R a = R(alpha[rhs]);
     cplx<typename SpinTraits<SX>::R> vx[12];
@@ -189,7 +198,7 @@ __global__ void __launch_bounds__(256) k_cg_xr_t(FieldRef x, FieldRef p, FieldRe
     spin_store<SX, typename SpinTraits<SX>::R>(x, e, vx);
     spin_store<SR, typename SpinTraits<SR>::R>(r, e, vr);
   }
-  block_partial_d(n, partial, slot);
+  block_partial_d(in ? n : 0.0, partial, slot);
 }
 
 // The mixed CG's lagged solution update: the step x += alpha p of the
@@ -203,7 +212,7 @@ __global__ void __launch_bounds__(256) k_xpay_x_t(FieldRef p, FieldRef r, FieldR
   const double a = alpha[rhs];
   const bool act = active[rhs] != 0;
   if (!act && a == 0.0) return;
-  const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  ELEM_OR_RETURN
   using R = typename SpinTraits<SX>::R;
   cplx<typename SpinTraits<SP>::R> vp[12];
   spin_load<SP, typename SpinTraits<SP>::R>(p, e, vp);
@@ -247,7 +256,7 @@ __global__ void __launch_bounds__(256) k_xpay_x_s5(FieldRef p, FieldRef r, Field
   const double a = alpha[rhs];
   const bool act = active[rhs] != 0;
   if (!act && a == 0.0) return;
-  const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  ELEM_OR_RETURN
   using R = float;
   cplx<R> vp[12];
   spin_load<SpinH, R>(p, e, vp);
@@ -302,7 +311,7 @@ __global__ void __launch_bounds__(256) k_xpay_pair(FieldRef pin, FieldRef pout, 
   const double ao = XUPD ? a_old[rhs] : 0.0, an = XUPD ? a_new[rhs] : 0.0;
   const bool act = active[rhs] != 0;
   if (!act && ao == 0.0 && an == 0.0) return;
-  const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  ELEM_OR_RETURN
   using R = float;
   cplx<R> vi[12];
   spin_load<SpinH, R>(pin, e, vi);
@@ -371,7 +380,7 @@ __global__ void __launch_bounds__(256) k_cg_r_t(FieldRef r, FieldRef ap, const d
                                                 int64_t per_rhs, double* partial) {
   ELEM_SETUP
   double n = 0;
-  if (active[rhs]) {
+  if (in && active[rhs]) {
     using R = typename SpinTraits<SR>::R;
     const R a = R(alpha[rhs]);
     cplx<typename SpinTraits<SR>::R> vr[12];
@@ -385,7 +394,7 @@ __global__ void __launch_bounds__(256) k_cg_r_t(FieldRef r, FieldRef ap, const d
     }
     spin_store<SR, typename SpinTraits<SR>::R>(r, e, vr);
   }
-  block_partial_d(n, partial, slot);
+  block_partial_d(in ? n : 0.0, partial, slot);
 }
 
 // p = b p + r with p and r of different storage
@@ -393,7 +402,7 @@ template <typename SP, typename SR>
 __global__ void __launch_bounds__(256) k_xpay_t(FieldRef p, FieldRef r, const double* beta, const int* active, int64_t per_rhs) {
   const int rhs = blockIdx.y;
   if (!active[rhs]) return;
-  const int64_t e = (int64_t)rhs * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  ELEM_OR_RETURN
   using R = float;
   const R b = R(beta[rhs]);
   cplx<typename SpinTraits<SP>::R> vp[12];
@@ -409,7 +418,7 @@ __global__ void __launch_bounds__(256) k_xpay_t(FieldRef p, FieldRef r, const do
 // fill a field with zeros (used instead of memset so it can sit in captured graphs)
 template <typename S>
 __global__ void __launch_bounds__(256) k_zero(FieldRef x, int64_t per_rhs) {
-  const int64_t e = (int64_t)blockIdx.y * per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  ELEM_OR_RETURN
   using R = typename SpinTraits<S>::R;
   cplx<R> v[12];
 #pragma unroll
@@ -507,7 +516,7 @@ __global__ void __launch_bounds__(REDUCE_MAX) k_reduce_rhs(const double* partial
 }
 
 static inline dim3 egrid(int64_t per_rhs, int bs, int nrhs) {
-  return dim3((unsigned)(per_rhs / bs), (unsigned)nrhs);
+  return dim3((unsigned)((per_rhs + bs - 1) / bs), (unsigned)nrhs);
 }
 
 hipError_t blas_norm(int st, const FieldRef& x, int64_t per_rhs, int nrhs, int bs, double* partial, hipStream_t s) {

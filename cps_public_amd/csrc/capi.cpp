@@ -230,7 +230,7 @@ static int generic_apply(cps_hip_lattice* lat, const cps_hip_op* op, double* out
   double* part = nullptr;
   int bpr = 1;
   if (dot_prd) {
-    bpr = (op->kind == CPS_HIP_OP_MOBIUS) ? (int)(o.per_rhs / pick_block(o.per_rhs)) : hop_blocks_per_rhs(L, op);
+    bpr = (op->kind == CPS_HIP_OP_MOBIUS) ? block_count(o.per_rhs, pick_block(o.per_rhs)) : hop_blocks_per_rhs(L, op);
     rc = L.ensure_partial((int64_t)bpr * nrhs);
     if (rc) return rc;
     part = (double*)L.partial.p;
@@ -301,7 +301,7 @@ int cps_hip_matpc_dag_matpc_prec(cps_hip_lattice* lat, const cps_hip_op* op, int
   if (L.last_rc) return L.last_rc;
   if ((rc = upload(L, in, fi, o, 1, nrhs, 0))) return rc;
   CPSHIP_CHECK(convert_spinor(STORE_D, fi.ref(), st, si.ref(), n, L.stream));
-  const int bpr = (op->kind == CPS_HIP_OP_MOBIUS) ? (int)(o.per_rhs / pick_block(o.per_rhs)) : hop_blocks_per_rhs(L, op);
+  const int bpr = (op->kind == CPS_HIP_OP_MOBIUS) ? block_count(o.per_rhs, pick_block(o.per_rhs)) : hop_blocks_per_rhs(L, op);
   if ((rc = L.ensure_partial((int64_t)bpr * nrhs))) return rc;
   double* part = (double*)L.partial.p;
   if ((rc = apply_mdagm(L, op, hprec, so.ref(), si.ref(), t1.ref(), t2.ref(), part, nrhs))) return rc;

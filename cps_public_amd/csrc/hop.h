@@ -244,11 +244,17 @@ inline bool quad_setup(const HopParams& Q, int bs) {
   return Q.clov == CLOV_S5X && (Q.hc5 == 0.0 || 64 % Q.nb == 0);
 }
 
-// block size dividing n (a power of two, at most 256)
+// Threads per block for one thread per element of a rhs's n elements: the
+// largest power of two up to 256 that divides n, if that is a wavefront or
+// more.  Otherwise (4-D lattices with few factors of 2) 256, the last block
+// of every rhs in part idle: blocks that divide n would hold 8 to 32 threads
+// and leave most lanes of every wavefront empty.
 inline int pick_block(long long n) {
+  if (n % 64) return 256;
   int b = 256;
-  while (b > 1 && (n % b) != 0) b >>= 1;
+  while (n % b) b >>= 1;
   return b;
 }
+inline int block_count(long long n, int bs) { return (int)((n + bs - 1) / bs); }
 
 }  // namespace cpship

@@ -7,13 +7,18 @@ template <typename SIN, typename SOUT, typename LK, typename R>
 static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   const int64_t nelem = (int64_t)P.nrhs * P.nsites_out * P.nb;
   const int bs = P.block;
-  const int64_t nblk = (nelem + bs - 1) / bs;
+  const int64_t per_rhs = (int64_t)P.nsites_out * P.nb;
+  // element order: whole blocks per rhs, the last one in part idle where bs
+  // does not divide per_rhs
+  const bool packed = (P.flags & (HOP_SITEWAVE | HOP_RHSGROUP)) != 0;
+  if (per_rhs % bs && (P.flags & (HOP_SPATIAL | HOP_LDS_LINKS)) && !packed) return hipErrorInvalidValue;
+  if (packed && nelem % bs) return hipErrorInvalidValue;
+  const int64_t nblk = packed ? nelem / bs : (int64_t)block_count(per_rhs, bs) * P.nrhs;
   dim3 grid((unsigned)nblk), block(bs);
   // 32-bit block decomposition (hop_decode): per-rhs counts below 2^31
-  const int64_t per_rhs = (int64_t)P.nsites_out * P.nb;
-  if (per_rhs % bs || per_rhs >= (int64_t(1) << 31) || nblk >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+  if (per_rhs >= (int64_t(1) << 31) || nblk >= (int64_t(1) << 31)) return hipErrorInvalidValue;
   HopParams Q = P;
-  Q.bpr = (int)(per_rhs / bs);
+  Q.bpr = block_count(per_rhs, bs);
   Q.bpr_b = (int)(((int64_t)P.perm_S * P.nb) / bs);
   Q.nb_shift = (P.nb & (P.nb - 1)) == 0 ? __builtin_ctz((unsigned)P.nb) : -1;
   // partials per 64-site chunk: wavefront-aligned blocks, and a mapping that

@@ -670,7 +670,11 @@ __device__ __forceinline__ HopElem hop_decode(const HopParams& P, int64_t sb64, 
     E.rhs = sb / bpr;
     const int blk = sb - E.rhs * bpr;
     const int el0 = blk * (int)blockDim.x;
-    const int el = el0 + el_base;
+    int el = el0 + el_base;
+    if (el >= P.nsites_out * P.nb) {   // idle thread of a rhs's last block
+      el = 0;
+      E.rhs = P.nrhs;
+    }
     E.site = P.nb_shift >= 0 ? (el >> P.nb_shift) : el / P.nb;
     E.j = el - E.site * P.nb;
     E.pslot = sb;

@@ -54,8 +54,11 @@ template <typename S, int DAG>
 __global__ void __launch_bounds__(256) k_s5(S5Params P) {
   using R = typename SpinTraits<S>::R;
   const int rhs = blockIdx.y;
-  const int64_t e = (int64_t)rhs * P.per_rhs + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int s = (int)(e % P.ls);
+  const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool in = i0 < (uint32_t)P.per_rhs;   // the rhs's last block may be in part idle
+  const uint32_t i = in ? i0 : 0u;
+  const int64_t e = (int64_t)rhs * P.per_rhs + i;
+  const int s = (int)(i % (uint32_t)P.ls);
   const int64_t base = e - s;
   const R mass = R(P.mass);
   cplx<R> res[12];
@@ -91,11 +94,12 @@ __global__ void __launch_bounds__(256) k_s5(S5Params P) {
       res[k].im += xc * v[k].im;
     }
   }
-  spin_store<S, R>(P.out, e, res);
+  if (in) spin_store<S, R>(P.out, e, res);
   if (P.partial) {
     double n = 0;
+    if (in)
 #pragma unroll
-    for (int k = 0; k < 12; k++) n += double(res[k].re) * res[k].re + double(res[k].im) * res[k].im;
+      for (int k = 0; k < 12; k++) n += double(res[k].re) * res[k].re + double(res[k].im) * res[k].im;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
     __shared__ double red[16];
@@ -441,7 +445,7 @@ static int store_of(int hprec) { return hprec == PREC_D_D18 ? STORE_D : hprec ==
 
 static int launch_s5(Lattice& L, int hprec, S5Params& P) {
   const int bs = pick_block(P.per_rhs);
-  dim3 grid((unsigned)(P.per_rhs / bs), (unsigned)P.nrhs), block(bs);
+  dim3 grid((unsigned)block_count(P.per_rhs, bs), (unsigned)P.nrhs), block(bs);
   switch (store_of(hprec)) {
 #define CPSHIP_S5(S)                                                                   \
   if (P.dag) hipLaunchKernelGGL((k_s5<S, 1>), grid, block, 0, L.stream, P);            \

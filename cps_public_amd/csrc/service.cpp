@@ -196,7 +196,7 @@ struct Engine {
     }
     if (L.last_rc) return L.last_rc;
     bsb = pick_block(o.per_rhs);
-    bpr_blas = (int)(o.per_rhs / bsb);
+    bpr_blas = block_count(o.per_rhs, bsb);
     bpr_hop = hop_blocks_per_rhs(L, &op);
     if ((rc = L.ensure_partial((int64_t)std::max(bpr_blas, bpr_hop) * S))) return rc;
     part = (double*)L.partial.p;

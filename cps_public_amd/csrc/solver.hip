@@ -504,7 +504,7 @@ static bool rhsgroup_ok(const HopParams& P, int b, int flags) {
 // spinors, at most one link per thread to stage)
 static bool lds_links_ok(const HopParams& P, int b) {
   const bool half = P.prec == PREC_H_H12 || P.prec == PREC_H_B12 || P.prec == PREC_H_H18 || P.prec == PREC_H_B18;
-  if (!half || (P.clov != CLOV_NONE && P.clov != CLOV_S5X)) return false;
+  if (!half || (P.clov != CLOV_NONE && P.clov != CLOV_S5X) || ((int64_t)P.nsites_out * P.nb) % b) return false;
   return 8 * lds_sites_per_block(b, P.nb) <= b;
 }
 
@@ -652,7 +652,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
       if (P.partial && !hop_chunk_partials(P)) blocks.push_back(def_block);
       else
         for (int b : {64, 128, 256})
-          if (b <= def_block && per_rhs % b == 0) blocks.push_back(b);
+          if (b <= def_block && (per_rhs % b == 0 || per_rhs % 64)) blocks.push_back(b);
       hipEvent_t e0, e1;
       CPSHIP_CHECK(hipEventCreate(&e0));
       CPSHIP_CHECK(hipEventCreate(&e1));
@@ -745,7 +745,7 @@ int hop_blocks_per_rhs(Lattice& L, const cps_hip_op* op) {
   if (op_layout(op, L.ls, &o, L.g)) return 1;
   const long long n = (long long)o.nsites * o.nb;
   if (chunk_partials_shape(op->kind == CPS_HIP_OP_DWF ? KIND_DWF : KIND_WILSON, o.nb, n)) return (int)(n / 64);
-  return (int)(n / pick_block(n));
+  return block_count(n, pick_block(n));
 }
 
 // out = M in (dag 0) or M^dagger in (dag 1), M = 1 - kappa^2 D D
@@ -1024,7 +1024,7 @@ int cg_double_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int
   Field& t2 = L.field(S_T2, STORE_D, n);
   if (L.last_rc) return L.last_rc;
   const int bsb = pick_block(o.per_rhs);
-  const int bpr_blas = (int)(o.per_rhs / bsb);
+  const int bpr_blas = block_count(o.per_rhs, bsb);
   const int bpr_hop = hop_blocks_per_rhs(L, op);
   rc = L.ensure_partial((int64_t)std::max(bpr_blas, bpr_hop) * nrhs);
   if (rc) return rc;
@@ -1279,7 +1279,7 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
   Field& t2s = L.field(S_T2S, sps, n);
   if (L.last_rc) return L.last_rc;
   const int bsb = pick_block(o.per_rhs);
-  const int bpr_blas = (int)(o.per_rhs / bsb);
+  const int bpr_blas = block_count(o.per_rhs, bsb);
   const int bpr_hop = hop_blocks_per_rhs(L, op);
   rc = L.ensure_partial((int64_t)std::max(bpr_blas, bpr_hop) * nrhs);
   if (rc) return rc;
