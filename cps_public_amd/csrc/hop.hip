@@ -46,11 +46,11 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   if (P.rupd) {
     // the CG residual update instead of the store (CLOV_NRR), for the last hop
     // of M^dag: half-precision or FP64 hops with X, element or spatial order;
-    // the FP64 Wilson kind also in the rhs-group mapping
+    // the Wilson kind also in the rhs-group mapping
     constexpr bool D = std::is_same<SIN, SpinD>::value, H = std::is_same<SIN, SpinH>::value;
     const bool group = (P.flags & HOP_RHSGROUP) != 0;
     if (P.clov != CLOV_NONE || !P.dag || !P.X.data || !P.R.data || !P.ralpha || !P.ractive || P.m5post ||
-        (P.kind != KIND_DWF && !D) || (group && P.kind == KIND_DWF) ||
+        (group && P.kind == KIND_DWF) ||
         (P.flags & (HOP_SITEWAVE | HOP_LDS_LINKS | HOP_LINK_ROW)))
       return hipErrorInvalidValue;
     if constexpr (D || H) {
@@ -59,7 +59,7 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   else hipLaunchKernelGGL((k_hop<SIN, SOUT, LK, R, 1, KIND, false, CLOV_NRR, SW>), grid, block, 0, st, Q);
       if (P.kind == KIND_DWF) {
         CPSHIP_HOP_NRR(KIND_DWF, 0)
-      } else if constexpr (D) {
+      } else {
         if (group) { CPSHIP_HOP_NRR(KIND_WILSON, 3) } else { CPSHIP_HOP_NRR(KIND_WILSON, 0) }
       }
 #undef CPSHIP_HOP_NRR

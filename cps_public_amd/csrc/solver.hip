@@ -634,7 +634,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
     // order 245 us), and blocks of one wavefront where larger ones would leave
     // CUs idle.  FP64 residuals that do not stay in the 256 MB cache between
     // two kernels are stored around it.
-    if (P.rupd && P.prec == PREC_D_D18) {
+    if (P.rupd && P.clov == CLOV_NONE) {
       if (P.nb == 1 && hop_chunk_partials(P)) {
         if (per_rhs * P.nrhs < 256 * 256) best.block = 64;
         for (int G : {4, 2}) {
@@ -645,7 +645,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
           }
         }
       }
-      if (per_rhs * P.nrhs * 192 > (int64_t(32) << 20)) best.flags |= HOP_NT_STORE;
+      if (P.prec == PREC_D_D18 && per_rhs * P.nrhs * 192 > (int64_t(32) << 20)) best.flags |= HOP_NT_STORE;
     }
     if (tuning_enabled() && !P.rupd) {
       std::vector<int> blocks;
@@ -760,10 +760,9 @@ int apply_m(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& out, co
 
 // M^dag t3 = t3 - kappa^2 D^dag D^dag t3 (wilson_m.C:73-91, dwf_mdag.C:32-62)
 // with r -= alpha M^dag t3 and |r|^2 in the epilogue of the second hop
-// (CLOV_NRR): DWF in half precision and FP64, Wilson in FP64
+// (CLOV_NRR): Wilson and DWF, in half precision and FP64
 bool mdag_rupdate_ok(const cps_hip_op* op, int hprec) {
-  if (op->kind == CPS_HIP_OP_WILSON) return hprec == PREC_D_D18;
-  return op->kind == CPS_HIP_OP_DWF && hprec != PREC_F_F12;
+  return (op->kind == CPS_HIP_OP_WILSON || op->kind == CPS_HIP_OP_DWF) && hprec != PREC_F_F12;
 }
 
 int mdag_rupdate(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& r, const FieldRef& t3,
@@ -1340,9 +1339,9 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
   // takes 3.85 instead of 2.56 s.
   const bool clover_rih = lagged && op->kind == CPS_HIP_OP_CLOVER && sps == STORE_H && svec == STORE_H &&
                           tn.clover_r_in_hop != 0;
-  // DWF, FP16 directions and residual: the residual step in the epilogue of
-  // the second hop of M^dag (CPS_HIP_R_IN_HOP=0: a separate pass)
-  const bool dwf_rih = lagged && op->kind == CPS_HIP_OP_DWF && sps == STORE_H && svec == STORE_H &&
+  // Wilson and DWF, FP16 directions and residual: the residual step in the
+  // epilogue of the second hop of M^dag (CPS_HIP_R_IN_HOP=0: a separate pass)
+  const bool mdag_rih = lagged && mdag_rupdate_ok(op, hprec) && sps == STORE_H && svec == STORE_H &&
                        tn.r_in_hop != 0;
   Field& t3s = L.field_min(S_T3S, sps, n);
   if (L.last_rc) return L.last_rc;
@@ -1414,7 +1413,7 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
         CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_BETA, sw, L.stream));
         return 0;
       }
-      if (dwf_rih) {
+      if (mdag_rih) {
         // M p with |M p|^2, alpha, then r -= alpha M^dag (M p) with |r|^2
         int e = apply_m(L, op, hprec, t3s.ref(), pw, t1s.ref(), 0, part, nw);
         if (e) return e;
@@ -1462,7 +1461,7 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
                                        bsb, L.stream));
       else
         CPSHIP_CHECK(blas_xpay_mixed(sps, psw, svec, rsw, sw.beta, sw.active, o.per_rhs, nw, bsb, L.stream));
-      if (clover_rih || dwf_rih) return opstep(psw);
+      if (clover_rih || mdag_rih) return opstep(psw);
       if (r_in_hop) {
         // M p with |M p|^2, alpha, then r -= alpha M^dag (M p) with |r|^2
         int e = mobius_m(L, op, hprec, t3s.ref(), psw, t1s.ref(), t2s.ref(), 0, part, nw, true);
