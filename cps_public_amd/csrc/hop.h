@@ -178,13 +178,9 @@ inline size_t lds_link_bytes(int sites) { return (size_t)sites * (LDS_SITE_WORDS
 
 // Shapes whose |out|^2 partials are per 64-element chunk rather than per
 // block: Wilson kind with one element per site (the 4-D Wilson and clover
-// operators) and a whole number of chunks per rhs
-inline bool chunk_partials_shape(int kind, int nb, long long per_rhs) {
-  return kind == KIND_WILSON && nb == 1 && per_rhs % 64 == 0;
-}
-inline bool hop_chunk_partials(const HopParams& P) {
-  return P.partial && chunk_partials_shape(P.kind, P.nb, (long long)P.nsites_out * P.nb);
-}
+// operators); the last chunk of a rhs may be a part
+inline bool chunk_partials_shape(int kind, int nb) { return kind == KIND_WILSON && nb == 1; }
+inline bool hop_chunk_partials(const HopParams& P) { return P.partial && chunk_partials_shape(P.kind, P.nb); }
 
 // HOP_RHSGROUP with HOP_SPATIAL: rhs groups swept together, so that each link
 // and clover term is fetched once for all of them, as long as the input
@@ -208,7 +204,9 @@ inline bool rhsgroup_setup(HopParams& Q, int bs) {
   if (Q.kind != KIND_WILSON || (Q.flags & (HOP_SITEWAVE | HOP_LDS_LINKS))) return false;
   if (Q.nb < 1 || (Q.nb & (Q.nb - 1)) || G * Q.nb > 64 || Q.nrhs % G || bs < 64 || bs % 64) return false;
   const int S = 64 / (G * Q.nb);
-  if (Q.nsites_out % ((bs / 64) * S)) return false;
+  // several elements per site: whole blocks; one: the last block of a group
+  // may be in part idle
+  if (Q.nb > 1 && Q.nsites_out % ((bs / 64) * S)) return false;
   if (Q.flags & HOP_SPATIAL) {
     // whole blocks (and, with partials, whole chunks) per spatial block
     if (!Q.perm || (Q.flags & HOP_NO_XCD_REMAP) || Q.perm_S % ((bs / 64) * S) || (Q.partial && Q.perm_S % 64))

@@ -10,10 +10,19 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   const int64_t per_rhs = (int64_t)P.nsites_out * P.nb;
   // element order: whole blocks per rhs, the last one in part idle where bs
   // does not divide per_rhs
-  const bool packed = (P.flags & (HOP_SITEWAVE | HOP_RHSGROUP)) != 0;
-  if (per_rhs % bs && (P.flags & (HOP_SPATIAL | HOP_LDS_LINKS)) && !packed) return hipErrorInvalidValue;
-  if (packed && nelem % bs) return hipErrorInvalidValue;
-  const int64_t nblk = packed ? nelem / bs : (int64_t)block_count(per_rhs, bs) * P.nrhs;
+  if (per_rhs % bs && (P.flags & (HOP_SPATIAL | HOP_LDS_LINKS)) &&
+      !(P.flags & (HOP_SITEWAVE | HOP_RHSGROUP)))
+    return hipErrorInvalidValue;
+  int64_t nblk = (int64_t)block_count(per_rhs, bs) * P.nrhs;
+  if (P.flags & HOP_RHSGROUP) {
+    // rhs groups times blocks of W S sites
+    const int G = hop_rhsgroup_G(P.flags);
+    if (P.nrhs % G || bs % G || P.nb < 1) return hipErrorInvalidValue;
+    nblk = (int64_t)block_count(per_rhs, bs / G) * (P.nrhs / G);
+  } else if (P.flags & HOP_SITEWAVE) {
+    if (nelem % bs) return hipErrorInvalidValue;
+    nblk = nelem / bs;
+  }
   dim3 grid((unsigned)nblk), block(bs);
   // 32-bit block decomposition (hop_decode): per-rhs counts below 2^31
   if (per_rhs >= (int64_t(1) << 31) || nblk >= (int64_t(1) << 31)) return hipErrorInvalidValue;

@@ -486,14 +486,15 @@ __device__ __forceinline__ void block_partial(R v, double* partial, int64_t slot
 __device__ __forceinline__ void chunk_partial_elem(const HopParams& P, int rhs, int site, double v) {
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m);
-  if ((threadIdx.x & 63) == 0) P.partial[(int64_t)rhs * (P.nsites_out >> 6) + (site >> 6)] = v;
+  // (a wavefront past the last element holds no chunk)
+  if ((threadIdx.x & 63) == 0 && rhs < P.nrhs) P.partial[(int64_t)rhs * ((P.nsites_out + 63) >> 6) + (site >> 6)] = v;
 }
 
 // HOP_RHSGROUP (lane = g S + q, S = 64 / G sites of rhs g): the butterfly
 // over the S lanes of each rhs gives the first log2 S levels of that tree;
 // the G wavefronts of a chunk (in one block, G <= W) then combine pairwise,
 // (a0 + a1) + (a2 + a3), as the remaining levels.
-__device__ __forceinline__ void chunk_partial_rhsgroup(const HopParams& P, int rhs, int64_t pslot, double v) {
+__device__ __forceinline__ void chunk_partial_rhsgroup(const HopParams& P, int rhs0, int64_t pslot, double v) {
   __shared__ double cred[16];
   const int s_shift = 6 - P.rg_shift, S = 1 << s_shift, G = 1 << P.rg_shift;
   for (int m = 1; m < S; m <<= 1) v += __shfl_xor(v, m);
@@ -506,7 +507,8 @@ __device__ __forceinline__ void chunk_partial_rhsgroup(const HopParams& P, int r
     // G is 2 or 4 (G <= W <= 4)
     const double* cw = cred + c * G * G + g;
     const double sum = G == 2 ? cw[0] + cw[G] : (cw[0] + cw[G]) + (cw[2 * G] + cw[3 * G]);
-    P.partial[(int64_t)((rhs & ~(G - 1)) + g) * (P.nsites_out >> 6) + pslot + c] = sum;
+    const int64_t nchunk = (P.nsites_out + 63) >> 6;
+    if (pslot + c < nchunk) P.partial[(rhs0 + g) * nchunk + pslot + c] = sum;
   }
 }
 
@@ -547,6 +549,7 @@ template <> struct HopWaves<SpinH> { static constexpr int value = CPSHIP_HOP_WAV
 struct HopElem {
   int rhs, site, j;
   int64_t pslot;   // rhs * blocks_per_rhs + sub-block within the rhs
+  int rhs0;        // HOP_RHSGROUP: first rhs of the wavefront's group
   // site range of the block (element mapping): sites qb .. qb+nsl-1 in site
   // order (through the spatial block b's permutation for HOP_SPATIAL); the
   // element's site is qb + sl
@@ -622,15 +625,20 @@ __device__ __forceinline__ HopElem hop_decode_rhsgroup(const HopParams& P, int64
     sblk = rem / cnt;
     rg = tile * P.rg_tile + rem - sblk * cnt;
   } else {
-    const int per_g = P.nsites_out / (W << s_shift);
+    const int per_g = (P.nsites_out + (W << s_shift) - 1) / (W << s_shift);
     rg = sb / per_g;
     sblk = sb - rg * per_g;
   }
   const int gq = lane >> P.nb_shift;
   const int g = gq >> s_shift;
   E.j = lane & (P.nb - 1);
-  E.rhs = (rg << P.rg_shift) + g;
-  const int q = ((sblk * W + w) << s_shift) + (gq - (g << s_shift));
+  E.rhs0 = rg << P.rg_shift;
+  E.rhs = E.rhs0 + g;
+  int q = ((sblk * W + w) << s_shift) + (gq - (g << s_shift));
+  if (q >= P.nsites_out) {   // idle thread of a group's last block
+    q = 0;
+    E.rhs = P.nrhs;
+  }
   E.site = (P.flags & HOP_SPATIAL) ? (int)P.perm[(int64_t)b * P.perm_S + q] : q;
   // partials (one element per site): the block's first chunk of 64 sites in
   // the order of the sweep
@@ -1175,7 +1183,7 @@ __global__ void __launch_bounds__(256, HopWaves<SIN>::value) k_hop(HopParams P) 
       P, E, N, reinterpret_cast<uint32_t*>(hop_lds_area));
   if (P.partial) {
     if (!P.chunk_part) block_partial<double>(nrm, P.partial, E.pslot);
-    else if constexpr (SW == 3) chunk_partial_rhsgroup(P, E.rhs, E.pslot, nrm);
+    else if constexpr (SW == 3) chunk_partial_rhsgroup(P, E.rhs0, E.pslot, nrm);
     else chunk_partial_elem(P, E.rhs, E.site, nrm);
   }
 }

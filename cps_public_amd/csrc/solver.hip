@@ -629,14 +629,18 @@ int tuned_launch(Lattice& L, HopParams& P) {
     if (quad) best.flags = HOP_QUAD | (spatial_ok(L, P, def_block) ? HOP_SPATIAL : 0);
     // a launch that updates a field in place (rupd) is never timed on the
     // live data: it keeps the fixed order of launches with partials.  One
-    // element per site: the rhs groups, which measured best wherever they
-    // divide the rhs (FP64 16^3x32 Wilson, 12 rhs: G = 4 146, 2 172, element
-    // order 245 us), and blocks of one wavefront where larger ones would leave
-    // CUs idle.  FP64 residuals that do not stay in the 256 MB cache between
-    // two kernels are stored around it.
+    // element per site: from 2^18 elements on the rhs groups, which share link
+    // loads that no cache holds by then (FP64 16^3x32 Wilson, 12 rhs: G = 4
+    // 146, 2 172, element order 245 us); below it blocks dealt over the XCDs
+    // in hardware order (10x12x14x18, 12 rhs: 52 us against 60 in XCD ranges
+    // and 55 in groups), of one wavefront where larger ones would leave CUs
+    // idle.  FP64 residuals that do not stay in the 256 MB cache between two
+    // kernels are stored around it.
     if (P.rupd && P.clov == CLOV_NONE) {
-      if (P.nb == 1 && hop_chunk_partials(P)) {
+      if (P.nb == 1 && per_rhs * P.nrhs < (1 << 18)) {
         if (per_rhs * P.nrhs < 256 * 256) best.block = 64;
+        best.flags = HOP_NO_XCD_REMAP;
+      } else if (P.nb == 1) {
         for (int G : {4, 2}) {
           const int f = HOP_RHSGROUP | ((G >> 2) << 6);
           if (rhsgroup_ok(P, best.block, f)) {
@@ -744,7 +748,7 @@ int hop_blocks_per_rhs(Lattice& L, const cps_hip_op* op) {
   OpLayout o;
   if (op_layout(op, L.ls, &o, L.g)) return 1;
   const long long n = (long long)o.nsites * o.nb;
-  if (chunk_partials_shape(op->kind == CPS_HIP_OP_DWF ? KIND_DWF : KIND_WILSON, o.nb, n)) return (int)(n / 64);
+  if (chunk_partials_shape(op->kind == CPS_HIP_OP_DWF ? KIND_DWF : KIND_WILSON, o.nb)) return block_count(n, 64);
   return block_count(n, pick_block(n));
 }
 
