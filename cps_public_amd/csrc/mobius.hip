@@ -28,6 +28,11 @@ struct S5Params {
   int dag, ls, nrhs;
   int64_t per_rhs;  // Vcb*Ls
   double* partial;
+  // RU: out is not stored; instead R -= ralpha[rhs] out for the rhs with
+  // ractive[rhs], and the partials are |R|^2
+  FieldRef R;
+  const double* ralpha;
+  const int* ractive;
 };
 
 // value of the CPS shift term (P+ from s-1, P- from s+1 for dag 0; exchanged
@@ -50,7 +55,7 @@ __device__ __forceinline__ void s5_term(const FieldRef& f, int64_t base, int s, 
   }
 }
 
-template <typename S, int DAG>
+template <typename S, int DAG, bool RU>
 __global__ void __launch_bounds__(256) k_s5(S5Params P) {
   using R = typename SpinTraits<S>::R;
   const int rhs = blockIdx.y;
@@ -94,10 +99,27 @@ __global__ void __launch_bounds__(256) k_s5(S5Params P) {
       res[k].im += xc * v[k].im;
     }
   }
-  if (in) spin_store<S, R>(P.out, e, res);
+  bool counts = in;
+  if constexpr (RU) {
+    // the CG step r -= alpha (M^dag M p), with M^dag M p in the arithmetic's precision
+    counts = in && P.ractive[rhs];
+    if (counts) {
+      const R al = R(P.ralpha[rhs]);
+      cplx<R> v[12];
+      spin_load<S, R>(P.R, e, v);
+#pragma unroll
+      for (int k = 0; k < 12; k++) {
+        res[k].re = v[k].re - al * res[k].re;
+        res[k].im = v[k].im - al * res[k].im;
+      }
+      spin_store<S, R>(P.R, e, res);
+    }
+  } else {
+    if (in) spin_store<S, R>(P.out, e, res);
+  }
   if (P.partial) {
     double n = 0;
-    if (in)
+    if (counts)
 #pragma unroll
       for (int k = 0; k < 12; k++) n += double(res[k].re) * res[k].re + double(res[k].im) * res[k].im;
 #pragma unroll
@@ -446,10 +468,16 @@ static int store_of(int hprec) { return hprec == PREC_D_D18 ? STORE_D : hprec ==
 static int launch_s5(Lattice& L, int hprec, S5Params& P) {
   const int bs = pick_block(P.per_rhs);
   dim3 grid((unsigned)block_count(P.per_rhs, bs), (unsigned)P.nrhs), block(bs);
+  if (P.ractive) {   // half precision, M^dag's last pass
+    if (store_of(hprec) != STORE_H || !P.dag || !P.ralpha || !P.R.data || !P.R.norm) return CPS_HIP_ERR_ARG;
+    hipLaunchKernelGGL((k_s5<SpinH, 1, true>), grid, block, 0, L.stream, P);
+    CPSHIP_CHECK(hipGetLastError());
+    return 0;
+  }
   switch (store_of(hprec)) {
-#define CPSHIP_S5(S)                                                                   \
-  if (P.dag) hipLaunchKernelGGL((k_s5<S, 1>), grid, block, 0, L.stream, P);            \
-  else hipLaunchKernelGGL((k_s5<S, 0>), grid, block, 0, L.stream, P);
+#define CPSHIP_S5(S)                                                                          \
+  if (P.dag) hipLaunchKernelGGL((k_s5<S, 1, false>), grid, block, 0, L.stream, P);            \
+  else hipLaunchKernelGGL((k_s5<S, 0, false>), grid, block, 0, L.stream, P);
     case STORE_D: CPSHIP_S5(SpinD) break;
     case STORE_F: CPSHIP_S5(SpinF) break;
     default: CPSHIP_S5(SpinH) break;
@@ -655,22 +683,44 @@ int mobius_m(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& out, c
 
 // r -= alpha M^dag t3 for the rhs with active set, and the partials |r|^2:
 // the second half of a CG iteration's M^dag M with the residual step in the
-// epilogue of M^dag's last hop (half precision, Ls 16: both fifth-dimension
-// stages run in hop epilogues, so M^dag is two hops)
+// last kernel of M^dag (half precision).  Ls 16: both fifth-dimension stages
+// run in hop epilogues, so M^dag is two hops; an Ls that does not divide 64:
+// the last kernel is k_s5.  Otherwise M^dag ends in a hop whose epilogue has
+// no such form.
+static bool rupdate_in_hop(const Lattice& L) { return L.ls == 16 && m5_fused_enabled() && s5_fused_enabled(); }
+
+bool mobius_rupdate_ok(const Lattice& L, int hprec) {
+  return store_of(hprec) == STORE_H && (rupdate_in_hop(L) || L.ls > 64 || 64 % L.ls != 0);
+}
+
 int mobius_mdag_rupdate(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& r, const FieldRef& t3,
                         const FieldRef& t1, const FieldRef& t2, const double* alpha, const int* active,
                         double* partial, int nrhs) {
-  (void)t1;
-  if (store_of(hprec) != STORE_H || L.ls != 16 || !m5_fused_enabled() || !s5_fused_enabled()) return CPS_HIP_ERR_ARG;
+  if (!mobius_rupdate_ok(L, hprec)) return CPS_HIP_ERR_ARG;
   double kb, kc;
   mobius_kappas(op, &kb, &kc);
   const double ratio = kb / kc;
-  const M5Post m5{ratio, op->mass, op->mobius_b, op->mobius_c};
-  int rc = hop4(L, hprec, t2, t3, 0, 1, -kb, nrhs, false, nullptr, 0.0, 0.0, nullptr, 1.0, 0.0, &m5);
-  if (rc) return rc;
-  const RUpdate ru{r, alpha, active};
-  return hop4(L, hprec, r, t2, 1, 1, kb, nrhs, true, &t3, ratio, op->mass, partial, op->mobius_b, op->mobius_c,
-              nullptr, &ru);
+  int rc;
+  if (rupdate_in_hop(L)) {
+    const M5Post m5{ratio, op->mass, op->mobius_b, op->mobius_c};
+    if ((rc = hop4(L, hprec, t2, t3, 0, 1, -kb, nrhs, false, nullptr, 0.0, 0.0, nullptr, 1.0, 0.0, &m5))) return rc;
+    const RUpdate ru{r, alpha, active};
+    return hop4(L, hprec, r, t2, 1, 1, kb, nrhs, true, &t3, ratio, op->mass, partial, op->mobius_b, op->mobius_c,
+                nullptr, &ru);
+  }
+  // as mobius_m (dag 1)
+  if ((rc = hop4(L, hprec, t1, t3, 0, 1, -kb, nrhs))) return rc;
+  if ((rc = launch_m5inv(L, hprec, t1, 1, ratio, op->mass, nrhs, &t2, S5_BEFORE, op->mobius_b, op->mobius_c)))
+    return rc;
+  if ((rc = hop4(L, hprec, t1, t2, 1, 1, kb, nrhs))) return rc;
+  S5Params P = s5_base(L, op, 1, nrhs);
+  P.A = t1; P.a1 = 1; P.b1 = op->mobius_b; P.c1 = op->mobius_c;
+  P.B = t3; P.a2 = 1; P.b2 = 1; P.c2 = ratio;
+  P.partial = partial;
+  P.R = r;
+  P.ralpha = alpha;
+  P.ractive = active;
+  return launch_s5(L, hprec, P);
 }
 
 // mobius_mdagm (mobius_mdagm.C:33-60): t3 = M in, |t3|^2, out = M^dag t3.

@@ -1331,10 +1331,11 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
   // (CPS_HIP_S5_XPAY=0: the operator computes it)
   const bool s5_in_xpay = lagged && tn.s5_xpay != 0 && op->kind == CPS_HIP_OP_MOBIUS && sps == STORE_H &&
                           xvec == STORE_F && L.ls == 16;
-  // with it, the residual step r -= alpha A p runs in the epilogue of the
-  // last hop of M^dag (alpha is known after the first half of M^dag M), so A p
-  // is never stored (CPS_HIP_R_IN_HOP=0: a separate pass)
-  const bool r_in_hop = s5_in_xpay && svec == STORE_H && tn.r_in_hop != 0;
+  // Moebius: the residual step r -= alpha A p runs in the last kernel of M^dag
+  // where that has such a form (alpha is known after the first half of M^dag
+  // M), so A p is never stored (CPS_HIP_R_IN_HOP=0: a separate pass)
+  const bool r_in_hop = lagged && op->kind == CPS_HIP_OP_MOBIUS && svec == STORE_H && tn.r_in_hop != 0 &&
+                        (L.ls != 16 || s5_in_xpay) && mobius_rupdate_ok(L, hprec);
   // clover, FP16 directions and residual, on request
   // (CPS_HIP_CLOVER_R_IN_HOP=1): likewise the residual step in the epilogue
   // of the last hop of MatPcDag, after the alpha of the first half.  Off by
@@ -1409,7 +1410,7 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
       }
       if (r_in_hop) {
         // M p with |M p|^2, alpha, then r -= alpha M^dag (M p) with |r|^2
-        int e = mobius_m(L, op, hprec, t3s.ref(), pw, t1s.ref(), t2s.ref(), 0, part, nw, true);
+        int e = mobius_m(L, op, hprec, t3s.ref(), pw, t1s.ref(), t2s.ref(), 0, part, nw, s5_in_xpay);
         if (e) return e;
         CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_ALPHA, sw, L.stream));
         e = mobius_mdag_rupdate(L, op, hprec, rsw, t3s.ref(), t1s.ref(), t2s.ref(), sw.alpha, sw.active, part, nw);
@@ -1468,7 +1469,7 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
       if (clover_rih || mdag_rih) return opstep(psw);
       if (r_in_hop) {
         // M p with |M p|^2, alpha, then r -= alpha M^dag (M p) with |r|^2
-        int e = mobius_m(L, op, hprec, t3s.ref(), psw, t1s.ref(), t2s.ref(), 0, part, nw, true);
+        int e = mobius_m(L, op, hprec, t3s.ref(), psw, t1s.ref(), t2s.ref(), 0, part, nw, s5_in_xpay);
         if (e) return e;
         CPSHIP_CHECK(reduce_rhs(part, bpr_hop, nw, nullptr, RED_CG_ALPHA, sw, L.stream));
         e = mobius_mdag_rupdate(L, op, hprec, rsw, t3s.ref(), t1s.ref(), t2s.ref(), sw.alpha, sw.active, part, nw);

@@ -47,3 +47,29 @@ def test_default_half_hop_matches_element_mapping(monkeypatch, kind, ls, L, nrhs
     assert err[""] < 1.1 * err["element"], err
     bound = 5e-3 if prec == C.PREC_MIXED_HALF else 3e-2
     assert err[""] < bound and np.allclose(res[""][1], norms, rtol=bound, atol=0)
+
+
+@pytest.mark.parametrize("ls,nrhs", [(6, 1), (12, 3), (20, 2), (8, 1)])
+def test_mobius_residual_step_in_last_kernel(monkeypatch, ls, nrhs):
+    """Mixed Moebius solves with the residual step in M^dag's last kernel (an
+    Ls that does not divide 64) and as a pass of its own (CPS_HIP_R_IN_HOP=0;
+    8 always): A p is rounded to FP16 in between only in the second, so the
+    residual histories differ in rounding and both meet the FP64 stopping
+    rule; the solutions then agree within the tolerance times the condition of
+    M^dag M, below 1e4 at this mass."""
+    L = [4, 6, 4, 8]
+    op = C.make_op(C.OP_MOBIUS, mass=0.1, m5=1.8, b=1.5, c=0.5)
+    n = int(np.prod(L)) // 2 * ls
+    src = np.concatenate([F.gaussian_fermion(n, 350 + k) for k in range(nrhs)])
+    arg = C.make_cg_arg(1e-11, 5000, precision=C.PREC_MIXED_HALF)
+    lat = C.Lattice(L, ls, (0, 0, 0, 1))
+    lat.import_gauge(wilson_gauge(L, 0.2, 349))
+    sol, its = {}, {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("CPS_HIP_R_IN_HOP", mode)
+        sol[mode], res = lat.invcg(op, src, arg, nrhs=nrhs)
+        its[mode] = [r.iterations for r in res]
+        assert max(r.true_res for r in res) <= 1e-11
+    assert rel(sol["1"], sol["0"]) < 1e-7
+    assert max(abs(a - b) / b for a, b in zip(its["1"], its["0"])) < 0.15, its
+    lat.close()
