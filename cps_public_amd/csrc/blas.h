@@ -29,6 +29,12 @@ hipError_t blas_redot(int st, const FieldRef& x, const FieldRef& y, int64_t per_
                       double* partial, hipStream_t s);
 hipError_t blas_sub_norm_d(const FieldRef& b, const FieldRef& a, const FieldRef& r, int64_t per_rhs, int nrhs, int bs,
                            double* partial, hipStream_t s);
+// r = b - a with |r|^2 in FP64, r stored in the format sr (FP32 or FP16)
+hipError_t blas_sub_norm(const FieldRef& b, const FieldRef& a, int sr, const FieldRef& r, int64_t per_rhs, int nrhs,
+                         int bs, double* partial, hipStream_t s);
+// y += x, x = 0 (x FP32 or FP16, y FP64)
+hipError_t blas_accumulate(int sx, const FieldRef& x, const FieldRef& y, int64_t per_rhs, int nrhs, int bs,
+                           hipStream_t s);
 hipError_t blas_cg_xr_d(const FieldRef& x, const FieldRef& p, const FieldRef& r, const FieldRef& ap, const CGScalars& cg,
                         int64_t per_rhs, int nrhs, int bs, double* partial, hipStream_t s);
 hipError_t blas_xpay(int st, const FieldRef& p, const FieldRef& r, const double* beta, const int* active,

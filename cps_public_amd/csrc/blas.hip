@@ -106,6 +106,46 @@ __global__ void __launch_bounds__(256) k_sub_norm_d(FieldRef b, FieldRef a, Fiel
   if (partial) block_partial_d(in ? n : 0.0, partial, slot);
 }
 
+// r = b - a in FP64 and |r|^2, r stored in the sloppy format only (a reliable
+// update needs no FP64 copy of it): 436 bytes an element (FP16) instead of the
+// 820 of an FP64 store and its conversion
+template <typename S>
+__global__ void __launch_bounds__(256) k_sub_norm_t(FieldRef b, FieldRef a, FieldRef r, int64_t per_rhs, double* partial) {
+  ELEM_SETUP
+  using R = typename SpinTraits<S>::R;
+  cplx<double> vb[12], va[12];
+  cplx<R> o[12];
+  spin_load<SpinD, double>(b, e, vb);
+  spin_load<SpinD, double>(a, e, va);
+  double n = 0;
+#pragma unroll
+  for (int c = 0; c < 12; c++) {
+    va[c] = cmk<double>(vb[c].re - va[c].re, vb[c].im - va[c].im);
+    n += va[c].re * va[c].re + va[c].im * va[c].im;
+    o[c] = cmk<R>(R(va[c].re), R(va[c].im));
+  }
+  if (in) spin_store<S, R>(r, e, o);
+  block_partial_d(in ? n : 0.0, partial, slot);
+}
+
+// y += x in FP64 (x sloppy), x = 0
+template <typename SX>
+__global__ void __launch_bounds__(256) k_accumulate(FieldRef x, FieldRef y, int64_t per_rhs) {
+  ELEM_OR_RETURN
+  using RX = typename SpinTraits<SX>::R;
+  cplx<RX> vx[12];
+  cplx<double> vy[12];
+  spin_load<SX, RX>(x, e, vx);
+  spin_load<SpinD, double>(y, e, vy);
+#pragma unroll
+  for (int k = 0; k < 12; k++) {
+    vy[k] = cmk<double>(vy[k].re + double(vx[k].re), vy[k].im + double(vx[k].im));
+    vx[k] = cmk<RX>(RX(0), RX(0));
+  }
+  spin_store<SpinD, double>(y, e, vy);
+  spin_store<SX, RX>(x, e, vx);
+}
+
 // x += a p ; r -= a Ap ; |r|^2   (inv_cg.C:340-349), skipped for inactive rhs
 __global__ void __launch_bounds__(256) k_cg_xr_d(FieldRef x, FieldRef p, FieldRef r, FieldRef ap,
                                                 const double* alpha, const int* active, int64_t per_rhs,
@@ -537,6 +577,25 @@ hipError_t blas_redot(int st, const FieldRef& x, const FieldRef& y, int64_t per_
 hipError_t blas_sub_norm_d(const FieldRef& b, const FieldRef& a, const FieldRef& r, int64_t per_rhs, int nrhs, int bs,
                            double* partial, hipStream_t s) {
   hipLaunchKernelGGL(k_sub_norm_d, egrid(per_rhs, bs, nrhs), dim3(bs), 0, s, b, a, r, per_rhs, partial);
+  return hipGetLastError();
+}
+
+hipError_t blas_sub_norm(const FieldRef& b, const FieldRef& a, int sr, const FieldRef& r, int64_t per_rhs, int nrhs,
+                         int bs, double* partial, hipStream_t s) {
+  const dim3 g = egrid(per_rhs, bs, nrhs), t(bs);
+  if (!partial) return hipErrorInvalidValue;
+  if (sr == STORE_F) hipLaunchKernelGGL(k_sub_norm_t<SpinF>, g, t, 0, s, b, a, r, per_rhs, partial);
+  else if (sr == STORE_H) hipLaunchKernelGGL(k_sub_norm_t<SpinH>, g, t, 0, s, b, a, r, per_rhs, partial);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+hipError_t blas_accumulate(int sx, const FieldRef& x, const FieldRef& y, int64_t per_rhs, int nrhs, int bs,
+                           hipStream_t s) {
+  const dim3 g = egrid(per_rhs, bs, nrhs), t(bs);
+  if (sx == STORE_F) hipLaunchKernelGGL(k_accumulate<SpinF>, g, t, 0, s, x, y, per_rhs);
+  else if (sx == STORE_H) hipLaunchKernelGGL(k_accumulate<SpinH>, g, t, 0, s, x, y, per_rhs);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

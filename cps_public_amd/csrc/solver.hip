@@ -1390,7 +1390,7 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
     if (win.update(live)) iter_graph.reset();
     const int lo = win.lo, nw = win.n();
     const FieldRef xw = rhs_view(x.ref(), o.per_rhs, lo), srcw = rhs_view(src.ref(), o.per_rhs, lo);
-    const FieldRef rw = rhs_view(r.ref(), o.per_rhs, lo), apw = rhs_view(ap.ref(), o.per_rhs, lo);
+    const FieldRef apw = rhs_view(ap.ref(), o.per_rhs, lo);
     const FieldRef xsw = rhs_view(xs.ref(), o.per_rhs, lo), rsw = rhs_view(rs.ref(), o.per_rhs, lo);
     const FieldRef psw = rhs_view(ps.ref(), o.per_rhs, lo), apsw = rhs_view(aps.ref(), o.per_rhs, lo);
     const CGScalars sw = scalars_view(cg.s, lo);
@@ -1514,13 +1514,11 @@ int cg_mixed_device(Lattice& L, const cps_hip_op* op, Field& x, Field& src, int 
       // (on the window: the rhs outside it have converged and keep x)
       if (lagged)   // the pending step x += alpha p of the last iteration
         CPSHIP_CHECK(blas_axpy(sps, psw, xvec, xsw, sw.alpha, 0.0, o.per_rhs, nw, bsb, L.stream));
-      CPSHIP_CHECK(blas_axpy(xvec, xsw, STORE_D, xw, nullptr, 1.0, o.per_rhs, nw, bsb, L.stream));
-      CPSHIP_CHECK(blas_zero(xvec, xsw, o.per_rhs, nw, bsb, L.stream));
+      CPSHIP_CHECK(blas_accumulate(xvec, xsw, xw, o.per_rhs, nw, bsb, L.stream));
       rc = apply_mdagm(L, op, PREC_D_D18, apw, xw, t1.ref(), t2.ref(), nullptr, nw);
       if (rc) return rc;
-      CPSHIP_CHECK(blas_sub_norm_d(srcw, apw, rw, o.per_rhs, nw, bsb, part, L.stream));
+      CPSHIP_CHECK(blas_sub_norm(srcw, apw, svec, rsw, o.per_rhs, nw, bsb, part, L.stream));
       CPSHIP_CHECK(reduce_rhs(part, bpr_blas, nw, rr_true + lo, RED_PLAIN, sw, L.stream));
-      CPSHIP_CHECK(convert_spinor(STORE_D, rw, svec, rsw, o.per_rhs * nw, L.stream));
       CPSHIP_CHECK(blas_redot_mixed(svec, rsw, sps, psw, o.per_rhs, nw, bsb, part, L.stream));
       // <r, p> into alpha (rewritten by the next step)
       CPSHIP_CHECK(reduce_rhs(part, bpr_blas, nw, sw.alpha, RED_PLAIN, sw, L.stream));
