@@ -14,41 +14,78 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
+#include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
 namespace cpship {
 
-HostStager::~HostStager() {
-  for (hipEvent_t e : done)
-    if (e) (void)hipEventDestroy(e);
-  if (pinned) (void)hipHostFree(pinned);
-}
+namespace {
 
-bool HostStager::ready() {
-  if (pinned) return true;
-  for (hipEvent_t& e : done)
-    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+struct Ring {
+  char* pinned = nullptr;   // WORKERS * BUFS chunks
+  hipEvent_t done[HostStager::WORKERS * HostStager::BUFS] = {};
+  int device = 0;
+  ~Ring() {
+    for (hipEvent_t e : done)
+      if (e) (void)hipEventDestroy(e);
+    if (pinned) (void)hipHostFree(pinned);
+  }
+};
+
+constexpr size_t MAX_IDLE = 2;
+std::mutex pool_mu;
+// (never destroyed: at exit the runtime may be gone before it)
+std::vector<std::unique_ptr<Ring>>& idle = *new std::vector<std::unique_ptr<Ring>>;
+int owners = 0;
+
+// a ring of the current device, or nullptr
+std::unique_ptr<Ring> take_ring() {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return nullptr;
+  {
+    std::lock_guard<std::mutex> lk(pool_mu);
+    for (size_t k = 0; k < idle.size(); k++)
+      if (idle[k]->device == device) {
+        std::unique_ptr<Ring> r = std::move(idle[k]);
+        idle.erase(idle.begin() + (long)k);
+        return r;
+      }
+  }
+  std::unique_ptr<Ring> r(new (std::nothrow) Ring);
+  if (!r) return nullptr;
+  r->device = device;
+  for (hipEvent_t& e : r->done)
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
       e = nullptr;
       (void)hipGetLastError();
-      return false;
+      return nullptr;
     }
   void* p = nullptr;
-  if (hipHostMalloc(&p, WORKERS * BUFS * CHUNK, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&p, HostStager::WORKERS * HostStager::BUFS * HostStager::CHUNK, hipHostMallocDefault) !=
+      hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return nullptr;
   }
-  pinned = static_cast<char*>(p);
-  return true;
+  r->pinned = static_cast<char*>(p);
+  return r;
+}
+
+// (one that the pool does not keep is freed on return)
+void give_ring(std::unique_ptr<Ring> r) {
+  std::lock_guard<std::mutex> lk(pool_mu);
+  if (owners > 0 && idle.size() < MAX_IDLE) idle.push_back(std::move(r));   // capacity reserved by the first owner
 }
 
 // Every chunk is taken by one worker; a worker's failure stops the others and
 // is returned.
-hipError_t HostStager::run(char* dev, char* host, size_t bytes, hipStream_t st, bool up) {
+hipError_t run(Ring& ring, char* dev, char* host, size_t bytes, hipStream_t st, bool up) {
+  constexpr int WORKERS = HostStager::WORKERS, BUFS = HostStager::BUFS;
+  constexpr size_t CHUNK = HostStager::CHUNK;
   const size_t nchunk = (bytes + CHUNK - 1) / CHUNK;
-  int device = 0;
-  hipError_t rc = hipGetDevice(&device);
-  if (rc != hipSuccess) return rc;
+  const int device = ring.device;
   std::atomic<size_t> next{0};
   std::atomic<int> failed{(int)hipSuccess};
   auto work = [&](int w) {
@@ -61,8 +98,8 @@ hipError_t HostStager::run(char* dev, char* host, size_t bytes, hipStream_t st, 
     hipEvent_t ev[BUFS];
     size_t at[BUFS], len[BUFS] = {};   // chunk in flight in each buffer (len 0: none)
     for (int b = 0; b < BUFS; b++) {
-      buf[b] = pinned + (size_t)(w * BUFS + b) * CHUNK;
-      ev[b] = done[w * BUFS + b];
+      buf[b] = ring.pinned + (size_t)(w * BUFS + b) * CHUNK;
+      ev[b] = ring.done[w * BUFS + b];
     }
     auto settle = [&](int b) {
       if (!len[b]) return true;
@@ -80,8 +117,10 @@ hipError_t HostStager::run(char* dev, char* host, size_t bytes, hipStream_t st, 
       if (up) std::memcpy(buf[b], host + off, n);
       if (!check(up ? hipMemcpyAsync(dev + off, buf[b], n, hipMemcpyHostToDevice, st)
                     : hipMemcpyAsync(buf[b], dev + off, n, hipMemcpyDeviceToHost, st)) ||
-          !check(hipEventRecord(ev[b], st)))
+          !check(hipEventRecord(ev[b], st))) {
+        (void)hipStreamSynchronize(st);   // a copy may be under way without its event
         break;
+      }
       at[b] = off;
       len[b] = n;
     }
@@ -100,12 +139,10 @@ hipError_t HostStager::run(char* dev, char* host, size_t bytes, hipStream_t st, 
   return (hipError_t)failed.load();
 }
 
-// Vectors below 32 MiB, which save less than the ring's allocation takes (0.7
-// ms, against 37 us a MiB) if a handle copies only one, and host memory that
-// the runtime knows (pinned, so that the DMA reads it directly) take a plain
-// copy.
-static bool worth_staging(const void* host, size_t bytes) {
-  if (bytes < 16 * HostStager::CHUNK) return false;
+// Vectors below 16 MiB, and host memory that the runtime knows (pinned, so
+// that the DMA reads it directly), take a plain copy.
+bool worth_staging(const void* host, size_t bytes) {
+  if (bytes < 8 * HostStager::CHUNK) return false;
   hipPointerAttribute_t a;
   if (hipPointerGetAttributes(&a, host) != hipSuccess) {
     (void)hipGetLastError();
@@ -114,17 +151,39 @@ static bool worth_staging(const void* host, size_t bytes) {
   return a.type == hipMemoryTypeUnregistered;
 }
 
+// the staged copy, if it is worth it and a ring is there
+bool staged(void* dev, void* host, size_t bytes, hipStream_t st, bool up, hipError_t* rc) {
+  if (!worth_staging(host, bytes)) return false;
+  std::unique_ptr<Ring> r = take_ring();
+  if (!r) return false;
+  *rc = run(*r, static_cast<char*>(dev), static_cast<char*>(host), bytes, st, up);
+  give_ring(std::move(r));
+  return true;
+}
+
+}  // namespace
+
+HostStager::HostStager() {
+  std::lock_guard<std::mutex> lk(pool_mu);
+  idle.reserve(MAX_IDLE);
+  owners++;
+}
+
+HostStager::~HostStager() {
+  std::lock_guard<std::mutex> lk(pool_mu);
+  if (--owners == 0) idle.clear();
+}
+
 hipError_t HostStager::to_device(void* dev, const void* host, size_t bytes, hipStream_t st) {
-  if (!worth_staging(host, bytes) || !ready()) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
-  return run(static_cast<char*>(dev), const_cast<char*>(static_cast<const char*>(host)), bytes, st, true);
+  hipError_t rc;
+  if (staged(dev, const_cast<void*>(host), bytes, st, true, &rc)) return rc;
+  return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
 }
 
 hipError_t HostStager::to_host(void* host, const void* dev, size_t bytes, hipStream_t st) {
   hipError_t rc;
-  if (!worth_staging(host, bytes) || !ready())
+  if (!staged(const_cast<void*>(dev), host, bytes, st, false, &rc))
     rc = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
-  else
-    rc = run(const_cast<char*>(static_cast<const char*>(dev)), static_cast<char*>(host), bytes, st, false);
   return rc == hipSuccess ? hipStreamSynchronize(st) : rc;
 }
 

@@ -6,14 +6,14 @@
 
 namespace cpship {
 
-// Ring of pinned buffers that large copies are staged through, allocated at
-// the first one and given back with its owner.  Not for concurrent use.
+// Staged copies for one owner.  A call takes a ring of pinned buffers from a
+// pool that all owners share (allocating one takes about 10 ms) and puts it
+// back when its transfers have ended; the pool keeps at most two idle rings
+// (64 MiB) and frees them with the last owner.  Safe from several threads.
 struct HostStager {
   static constexpr int WORKERS = 8, BUFS = 2;
   static constexpr size_t CHUNK = size_t(2) << 20;
-  char* pinned = nullptr;   // WORKERS * BUFS chunks
-  hipEvent_t done[WORKERS * BUFS] = {};
-  HostStager() = default;
+  HostStager();
   HostStager(const HostStager&) = delete;
   HostStager& operator=(const HostStager&) = delete;
   ~HostStager();
@@ -21,10 +21,6 @@ struct HostStager {
   // returns, and written when to_host returns (which waits for st).
   hipError_t to_device(void* dev, const void* host, size_t bytes, hipStream_t st);
   hipError_t to_host(void* host, const void* dev, size_t bytes, hipStream_t st);
-
- private:
-  bool ready();
-  hipError_t run(char* dev, char* host, size_t bytes, hipStream_t st, bool up);
 };
 
 }  // namespace cpship
