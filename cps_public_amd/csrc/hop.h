@@ -30,7 +30,7 @@ enum HopFlags {
                           // the 8 links of each of its sites in LDS once (f16
                           // words, third row rebuilt), and every thread keeps
                           // all 8 neighbour spinors in flight
-  HOP_RHSGROUP = 32,      // Wilson kind, nb a power of two, no partials: a
+  HOP_RHSGROUP = 32,      // Wilson kind, nb a power of two (partials per chunk): a
                           // wavefront computes S sites x G rhs (x nb slots),
                           // G = 2 << ((flags >> 6) & 3), so the G lanes of a
                           // site share its link and clover loads
