@@ -36,6 +36,9 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   if (Q.chunk_part && (bs % 64 || (P.flags & HOP_SITEWAVE) ||
                        ((P.flags & HOP_SPATIAL) && !(P.flags & HOP_RHSGROUP))))
     return hipErrorInvalidValue;
+  // partials per block: the reduction adds block_count(per_rhs,
+  // pick_block(per_rhs)) of them
+  if (P.partial && !Q.chunk_part && bs != pick_block(per_rhs)) return hipErrorInvalidValue;
   const bool nt = (P.flags & HOP_NT_STORE) != 0;
   // HOP_LDS_LINKS: half-precision spinors, one link per thread to stage
   const bool lds = (P.flags & HOP_LDS_LINKS) != 0;

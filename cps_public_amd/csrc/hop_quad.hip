@@ -434,6 +434,8 @@ hipError_t launch_hop_quad(const HopParams& P, hipStream_t st) {
   const int bs = P.block;
   const int64_t per_rhs = (int64_t)P.nsites_out * P.nb;
   if (!quad_setup(P, bs) || !P.gauge.data) return hipErrorInvalidValue;
+  // the reduction adds the partials of default blocks
+  if (P.partial && bs != pick_block(per_rhs)) return hipErrorInvalidValue;
   HopParams Q = P;
   Q.bpr = (int)(per_rhs / bs);
   Q.bpr_b = (int)(((int64_t)P.perm_S * P.nb) / bs);

@@ -637,10 +637,12 @@ int tuned_launch(Lattice& L, HopParams& P) {
     // idle.  FP64 residuals that do not stay in the 256 MB cache between two
     // kernels are stored around it.
     if (P.rupd && P.clov == CLOV_NONE) {
-      if (P.nb == 1 && per_rhs * P.nrhs < (1 << 18)) {
+      // (chunk partials: block partials, as a domain-wall field of two slices
+      // has with one element per site too, are tied to the default block)
+      if (hop_chunk_partials(P) && per_rhs * P.nrhs < (1 << 18)) {
         if (per_rhs * P.nrhs < 256 * 256) best.block = 64;
         best.flags = HOP_NO_XCD_REMAP;
-      } else if (P.nb == 1) {
+      } else if (hop_chunk_partials(P)) {
         for (int G : {4, 2}) {
           const int f = HOP_RHSGROUP | ((G >> 2) << 6);
           if (rhsgroup_ok(P, best.block, f)) {
