@@ -93,6 +93,10 @@ int Lattice::init(const int node_sites[4], int ls_, const int bc[4]) {
   if ((rc = nbr_neg.ensure((size_t)2 * g.Vcb * sizeof(uint32_t)))) return rc;
   CPSHIP_CHECK(build_nbr(g, (uint4*)nbr.p, (uint32_t*)nbr_neg.p, stream));
   CPSHIP_CHECK(hipStreamSynchronize(stream));
+  // domain-wall hops with partials are swept in the spatial order from Ls 16
+  // on (order_rule), also by the call that may not allocate: its table is
+  // there from the start (the handle's first hop would build it otherwise)
+  if (ls >= 16 && ls % 2 == 0 && g.Vcb % 8 == 0 && (rc = ensure_perm()) && perm_state >= 0) return rc;
   return 0;
 }
 
@@ -473,6 +477,8 @@ extern "C" int cps_hip_set_tuning(const cps_hip_tuning* t) {
 
 namespace cpship {
 
+thread_local int tl_no_alloc = 0;
+
 static bool tuning_enabled() { return knob(&cps_hip_tuning::tune, "CPS_HIP_TUNE") != 0; }
 
 // whether a launch may use HOP_SPATIAL at block size b
@@ -480,7 +486,19 @@ static bool spatial_ok(Lattice& L, const HopParams& P, int b) {
   if (L.g.Vcb % 8) return false;
   const long long per_b = (long long)(L.g.Vcb / 8) * P.nb * (P.kind == KIND_DWF ? 2 : 1);
   if (per_b % b) return false;
-  return L.ensure_perm() == 0;
+  return tl_no_alloc ? L.perm_state > 0 : L.ensure_perm() == 0;
+}
+
+// Order of a launch that is not timed, and of every launch that writes
+// per-block reduction partials (whose sums must not depend on tuning):
+// spatial for the 5-D layouts (nb >= 8 slots per site) whenever the geometry
+// allows it, element order otherwise (with one site per lane the spatial
+// sweep is the slower order: 6.2 against 4.6 ms for the 32^3x64 clover hop
+// with 48 rhs).  Per-chunk partials are summed alike in every mapping: the
+// element order is their default and the rhs-group mapping a candidate.
+static int order_rule(Lattice& L, const HopParams& P, int b, bool quad) {
+  if (quad) return HOP_QUAD | (spatial_ok(L, P, b) ? HOP_SPATIAL : 0);
+  return P.nb >= 8 && spatial_ok(L, P, b) ? HOP_SPATIAL : 0;
 }
 
 // whether a launch may use HOP_SITEWAVE at block size b (one site per
@@ -517,8 +535,6 @@ static int tune_report() { return knob(&cps_hip_tuning::tune_report, "CPS_HIP_TU
 static std::mutex tune_mu;
 static std::map<HopTuneKey, HopTuneVal> tune_cache;
 
-thread_local int tl_no_alloc = 0;
-
 int tuned_launch(Lattice& L, HopParams& P) {
   P.nbr = (const uint4*)L.nbr.p;
   P.nbr_neg = (const uint32_t*)L.nbr_neg.p;
@@ -547,9 +563,11 @@ int tuned_launch(Lattice& L, HopParams& P) {
   if (tl_no_alloc) {
     // no allocation and no timing (cps_hip_matpc_dag_matpc_noalloc): the
     // choice cached for this launch shape if it needs no table the handle
-    // lacks, else the default launch (results do not depend on the choice)
-    if (P.kind == KIND_WILSON && L.perm_state > 0) P.perm = (const uint32_t*)L.perm.p;
-    HopTuneVal chosen{def_block, 0, 0.0};
+    // lacks, else the default launch.  The same bits either way: an element's
+    // arithmetic does not depend on the choice, and the order of block
+    // partials is order_rule's in both
+    if (L.perm_state > 0) P.perm = (const uint32_t*)(P.kind == KIND_DWF ? L.perm5.p : L.perm.p);
+    HopTuneVal chosen{def_block, P.clov == CLOV_KS ? 0 : order_rule(L, P, def_block, false), 0.0};
     if (P.clov != CLOV_KS) {
       const HopTuneKey key{P.kind, P.prec, P.dag, P.nb, P.nsites_out, P.nrhs, P.partial != nullptr,
                            P.X.data != nullptr, P.clov + 16 * P.m5post + 32 * P.rupd,
@@ -617,16 +635,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
     }
   }
   if (!have) {
-    // launches that write per-block reduction partials use a fixed order
-    // (results do not depend on tuning): spatial for the 5-D layouts (nb >= 8
-    // slots per site) whenever the geometry allows it, element order
-    // otherwise (with one site per lane the spatial sweep is the slower
-    // order: 6.2 against 4.6 ms for the 32^3x64 clover hop with 48 rhs); with
-    // per-chunk partials the element order is the default and the rhs-group
-    // mapping a candidate
-    HopTuneVal best{def_block, (P.nb >= 8 && spatial_ok(L, P, def_block)) ? HOP_SPATIAL : 0,
-                    0.0};
-    if (quad) best.flags = HOP_QUAD | (spatial_ok(L, P, def_block) ? HOP_SPATIAL : 0);
+    HopTuneVal best{def_block, order_rule(L, P, def_block, quad), 0.0};
     // a launch that updates a field in place (rupd) is never timed on the
     // live data: it keeps the fixed order of launches with partials.  One
     // element per site: from 2^18 elements on the rhs groups, which share link

@@ -52,3 +52,22 @@ def test_noalloc_refuses_beyond_scratch():
         lat.mdagm_noalloc(op, src, nrhs=nrhs)
     assert e.value.code == C.ERR_TOO_LARGE
     lat.close()
+
+
+@pytest.mark.parametrize("L,ls", [([8, 8, 8, 4], 16), ([4, 8, 8, 8], 24), ([6, 6, 6, 4], 16)])
+def test_noalloc_matches_spatial_order(L, ls):
+    """From Ls 16 on a domain-wall hop with |M in|^2 partials sweeps spatial
+    blocks where the lattice splits into eight of them (the first two do): the
+    same bits from the call that may not allocate, as the handle's first call
+    and after one that chose its launches."""
+    nrhs = 8   # (a sum in another order often has the same bits)
+    op = C.make_op(C.OP_DWF, mass=0.02, m5=1.8)
+    lat = C.Lattice(L, ls, (0, 0, 0, 1))
+    lat.import_gauge(wilson_gauge(L, 0.2, 611))
+    src = np.concatenate([F.gaussian_fermion(lat._nreal(op) // 24, 640 + k) for k in range(nrhs)])
+    first, dfirst = lat.mdagm_noalloc(op, src, nrhs=nrhs)
+    ref, dref = lat.mdagm(op, src, nrhs=nrhs)
+    again, dagain = lat.mdagm_noalloc(op, src, nrhs=nrhs)
+    lat.close()
+    assert np.array_equal(first, ref) and np.array_equal(again, ref)
+    assert np.array_equal(dfirst, dref) and np.array_equal(dagain, dref)
