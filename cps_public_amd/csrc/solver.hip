@@ -535,6 +535,40 @@ static int tune_report() { return knob(&cps_hip_tuning::tune_report, "CPS_HIP_TU
 static std::mutex tune_mu;
 static std::map<HopTuneKey, HopTuneVal> tune_cache;
 
+// Launch of a residual step without a clover term (CLOV_NRR), in the mapping
+// that hop_mode asks for where there is one (the site-per-wavefront, LDS and
+// row mappings have no residual step).  One element per site: from 2^18
+// elements on the rhs groups, which share link loads that no cache holds by
+// then (FP64 16^3x32 Wilson, 12 rhs: G = 4 146, 2 172, element order 245 us);
+// below it blocks dealt over the XCDs in hardware order (10x12x14x18, 12 rhs:
+// 52 us against 60 in XCD ranges and 55 in groups), of one wavefront where
+// larger ones would leave CUs idle.  (Chunk partials: block partials, as a
+// domain-wall field of two slices has with one element per site too, are tied
+// to the default block.)  FP64 residuals that do not stay in the 256 MB cache
+// between two kernels are stored around it.
+static void rupd_rule(const HopParams& P, int mode, HopTuneVal& best) {
+  if (P.clov != CLOV_NONE) return;
+  const int64_t n = (int64_t)P.nsites_out * P.nb * P.nrhs;
+  if (hop_chunk_partials(P)) {
+    const bool small = n < (1 << 18);
+    if (small) {
+      if (n < 256 * 256) best.block = 64;
+      best.flags = HOP_NO_XCD_REMAP;
+    }
+    if (mode == 4 || (mode != 1 && !small))
+      for (int G : {4, 2}) {
+        const int f = HOP_RHSGROUP | ((G >> 2) << 6);
+        const int b = mode == 4 ? 256 : best.block;   // (256: a chunk's wavefronts in one block for both G)
+        if (rhsgroup_ok(P, b, f)) {
+          best.block = b;
+          best.flags = f;
+          break;
+        }
+      }
+  }
+  if (P.prec == PREC_D_D18 && n * 192 > (int64_t(32) << 20)) best.flags |= HOP_NT_STORE;
+}
+
 int tuned_launch(Lattice& L, HopParams& P) {
   P.nbr = (const uint4*)L.nbr.p;
   P.nbr_neg = (const uint32_t*)L.nbr_neg.p;
@@ -637,30 +671,12 @@ int tuned_launch(Lattice& L, HopParams& P) {
   if (!have) {
     HopTuneVal best{def_block, order_rule(L, P, def_block, quad), 0.0};
     // a launch that updates a field in place (rupd) is never timed on the
-    // live data: it keeps the fixed order of launches with partials.  One
-    // element per site: from 2^18 elements on the rhs groups, which share link
-    // loads that no cache holds by then (FP64 16^3x32 Wilson, 12 rhs: G = 4
-    // 146, 2 172, element order 245 us); below it blocks dealt over the XCDs
-    // in hardware order (10x12x14x18, 12 rhs: 52 us against 60 in XCD ranges
-    // and 55 in groups), of one wavefront where larger ones would leave CUs
-    // idle.  FP64 residuals that do not stay in the 256 MB cache between two
-    // kernels are stored around it.
-    if (P.rupd && P.clov == CLOV_NONE) {
-      // (chunk partials: block partials, as a domain-wall field of two slices
-      // has with one element per site too, are tied to the default block)
-      if (hop_chunk_partials(P) && per_rhs * P.nrhs < (1 << 18)) {
-        if (per_rhs * P.nrhs < 256 * 256) best.block = 64;
-        best.flags = HOP_NO_XCD_REMAP;
-      } else if (hop_chunk_partials(P)) {
-        for (int G : {4, 2}) {
-          const int f = HOP_RHSGROUP | ((G >> 2) << 6);
-          if (rhsgroup_ok(P, best.block, f)) {
-            best.flags = f;
-            break;
-          }
-        }
-      }
-      if (P.prec == PREC_D_D18 && per_rhs * P.nrhs * 192 > (int64_t(32) << 20)) best.flags |= HOP_NT_STORE;
+    // live data: it keeps the order of order_rule or rupd_rule
+    if (P.rupd) {
+      rupd_rule(P, mode, best);
+      if (tune_report() >= 1)
+        fprintf(stderr, "cps_hip rule: kind %d prec %d dag %d nb %d nsites %d nrhs %d clov %d residual step -> block %d flags %d\n",
+                P.kind, P.prec, P.dag, P.nb, P.nsites_out, P.nrhs, P.clov, best.block, best.flags);
     }
     if (tuning_enabled() && !P.rupd) {
       std::vector<int> blocks;

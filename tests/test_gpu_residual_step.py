@@ -1,5 +1,7 @@
 """The CG residual step in the epilogue of M^dag's last hop (CLOV_NRR), at the
 shapes whose launch rule differs from the other hops'."""
+import re
+
 import numpy as np
 import pytest
 
@@ -35,3 +37,50 @@ def test_two_slice_domain_wall_solve(oracle, L, nrhs):
         assert abs(res[k].iterations - it) <= 1
         assert res[k].true_res <= 1.1e-10 and rel(sol[part], x) < 1e-10
         assert hres[k].true_res <= 1e-10 and rel(half[part], x) < 4e-9
+
+
+def _flags(err):
+    """Launch flags of the residual steps reported on stderr."""
+    return [int(m) for m in re.findall(r"residual step -> block \d+ flags (\d+)", err)]
+
+
+RHSGROUP = 32   # HOP_RHSGROUP
+
+
+@pytest.mark.parametrize("L,nrhs", [([4, 4, 8, 4], 4), ([6, 6, 4, 6], 2), ([10, 4, 6, 6], 4), ([6, 10, 6, 6], 6),
+                                    ([14, 14, 10, 14], 14)])
+def test_residual_step_mappings(monkeypatch, capfd, L, nrhs):
+    """Wilson solves with the hops, the residual step among them, in element
+    order and with 4 or 2 rhs of a site in a wavefront (CPS_HIP_HOP_MODE):
+    whole and part chunks of 64 sites (256, 432, 720, 1080 and 13720 sites a
+    parity), rhs counts that 4 and that only 2 divides, the last one large
+    enough for streaming stores.  FP64: an element's arithmetic and the tree
+    of the partial sums are the same, so are all bits.  Half precision: the
+    two mappings are separate compilations (a few FP32 results round
+    differently), so twice the stopping rule's 1e-10 times the condition of
+    M^dag M, which is 20 for 6^4 and below 100 at this mass."""
+    u = wilson_gauge(L, 0.2, 71)
+    n = int(np.prod(L)) // 2
+    op = C.make_op(C.OP_WILSON, mass=0.1)
+    src = np.concatenate([F.gaussian_fermion(n, 72 + k) * (1.0 + k) for k in range(nrhs)])
+    monkeypatch.setenv("CPS_HIP_TUNE_REPORT", "1")
+    monkeypatch.setenv("CPS_HIP_RHS_WINDOW", "0")   # (a shrunk window may hold an odd count, which no group divides)
+    out = {}
+    for mode in ("element", "rhsgroup"):
+        monkeypatch.setenv("CPS_HIP_HOP_MODE", mode)
+        lat = C.Lattice(L, 1, (0, 0, 0, 1))
+        lat.import_gauge(u)
+        capfd.readouterr()
+        out[mode] = [lat.invcg(op, src, C.make_cg_arg(1e-10, 1000, precision=p), nrhs=nrhs)
+                     for p in (C.PREC_DOUBLE, C.PREC_MIXED_HALF)]
+        flags = _flags(capfd.readouterr().err)
+        assert flags and all(((f & RHSGROUP) != 0) == (mode == "rhsgroup") for f in flags), flags
+        lat.close()
+    (xe, re_), (xg, rg) = out["element"][0], out["rhsgroup"][0]
+    assert [r.iterations for r in re_] == [r.iterations for r in rg]
+    assert np.array_equal(xe, xg)
+    (xe, re_), (xg, rg) = out["element"][1], out["rhsgroup"][1]
+    assert max(r.true_res for r in re_ + rg) <= 1e-10
+    for k in range(nrhs):
+        part = slice(24 * n * k, 24 * n * (k + 1))
+        assert rel(xg[part], xe[part]) < 2e-8
