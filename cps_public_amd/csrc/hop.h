@@ -71,7 +71,7 @@ struct HopParams {
   // chunk_part (set by the launcher where hop_chunk_partials holds): one
   // partial per 64 consecutive elements of a rhs, summed as a pairwise tree
   // in element order (the same bits in every thread mapping that computes
-  // it), at partial[rhs * (elements per rhs / 64) + chunk]
+  // it), at partial[rhs * chunks per rhs + chunk]; the last may be a part
   int chunk_part;
   // clover epilogue (Wilson kind only): 0 none, CLOV_POST out = A (scale*hop),
   // CLOV_X out = xcoef*(A X) + kscale[set]*scale*hop, with A the clover set of
@@ -87,10 +87,11 @@ struct HopParams {
   // hop come from the neighbouring lanes of the site's 16-lane row (DPP
   // rotations) instead of loads and lane permutes
   int s5_row;
-  // rupd (with s5_row, or with the CLOV_X epilogue of FP16 hops): out is
-  // not stored; instead the CG residual R (FP16)
-  // of every rhs with ractive[rhs] becomes R - ralpha[rhs] * out, and the
-  // partials are |R|^2 (0 for the other rhs)
+  // rupd (with s5_row, with the CLOV_X epilogue of FP16 hops, or without a
+  // clover term for half-precision and FP64 hops): out is not stored; instead
+  // the CG residual R (in the hop's spinor format) of every rhs with
+  // ractive[rhs] becomes R - ralpha[rhs] * out, and the partials are |R|^2 (0
+  // for the other rhs)
   int rupd;
   FieldRef R;
   const double* ralpha;
@@ -208,9 +209,9 @@ inline bool rhsgroup_setup(HopParams& Q, int bs) {
   // may be in part idle
   if (Q.nb > 1 && Q.nsites_out % ((bs / 64) * S)) return false;
   if (Q.flags & HOP_SPATIAL) {
-    // whole blocks (and, with partials, whole chunks) per spatial block
-    if (!Q.perm || (Q.flags & HOP_NO_XCD_REMAP) || Q.perm_S % ((bs / 64) * S) || (Q.partial && Q.perm_S % 64))
-      return false;
+    // whole blocks per spatial block; chunk partials are of sites in element
+    // order
+    if (!Q.perm || (Q.flags & HOP_NO_XCD_REMAP) || Q.perm_S % ((bs / 64) * S) || Q.partial) return false;
   }
   Q.rg_shift = __builtin_ctz((unsigned)G);
   Q.rg_tile = rhsgroup_tile(Q, G);

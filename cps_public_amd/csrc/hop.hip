@@ -33,9 +33,7 @@ static hipError_t launch_t(const HopParams& P, hipStream_t st) {
   // partials per 64-site chunk: wavefront-aligned blocks, and a mapping that
   // keeps a chunk's sites in one block (element order or the rhs groups)
   Q.chunk_part = hop_chunk_partials(P) ? 1 : 0;
-  if (Q.chunk_part && (bs % 64 || (P.flags & HOP_SITEWAVE) ||
-                       ((P.flags & HOP_SPATIAL) && !(P.flags & HOP_RHSGROUP))))
-    return hipErrorInvalidValue;
+  if (Q.chunk_part && (bs % 64 || (P.flags & (HOP_SPATIAL | HOP_SITEWAVE)))) return hipErrorInvalidValue;
   // partials per block: the reduction adds block_count(per_rhs,
   // pick_block(per_rhs)) of them
   if (P.partial && !Q.chunk_part && bs != pick_block(per_rhs)) return hipErrorInvalidValue;

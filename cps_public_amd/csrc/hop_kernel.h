@@ -604,9 +604,9 @@ __device__ __forceinline__ void hop_block_sites(const HopParams& P, int el0, int
   E.sl = q - E.qb;
 }
 
-// HOP_RHSGROUP decode (Wilson kind, nb a power of two, no partials): lane =
-// (g S + q) nb + j with g < G rhs and q < S = 64 / (G nb) consecutive sites;
-// logical block sb = (rhs group, block of W S sites), W wavefronts per block
+// HOP_RHSGROUP decode (Wilson kind, nb a power of two): lane = (g S + q) nb +
+// j with g < G rhs and q < S = 64 / (G nb) consecutive sites; logical block
+// sb = (rhs group, block of W S sites), W wavefronts per block
 __device__ __forceinline__ HopElem hop_decode_rhsgroup(const HopParams& P, int64_t sb64, int64_t nsub64) {
   HopElem E;
   const int sb = (int)sb64;
@@ -640,9 +640,9 @@ __device__ __forceinline__ HopElem hop_decode_rhsgroup(const HopParams& P, int64
     E.rhs = P.nrhs;
   }
   E.site = (P.flags & HOP_SPATIAL) ? (int)P.perm[(int64_t)b * P.perm_S + q] : q;
-  // partials (one element per site): the block's first chunk of 64 sites in
-  // the order of the sweep
-  E.pslot = ((int64_t)b * P.perm_S + ((int64_t)(sblk * W) << s_shift)) >> 6;
+  // partials (one element per site, no spatial sweep): the block's first
+  // chunk of 64 sites
+  E.pslot = ((int64_t)(sblk * W) << s_shift) >> 6;
   E.qb = E.nsl = E.sl = E.b = 0;
   return E;
 }
