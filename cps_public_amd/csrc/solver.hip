@@ -526,6 +526,25 @@ static bool lds_links_ok(const HopParams& P, int b) {
   return 8 * lds_sites_per_block(b, P.nb) <= b;
 }
 
+// Flags of an untimed launch in the mapping that hop_mode asks for: `order`
+// (of order_rule) where that mapping is the element order or cannot run this
+// launch.  Rhs groups of 4 before those of 2, 8 and 16, swept by spatial
+// blocks where there are no partials.
+static int mapping_rule(Lattice& L, HopParams P, int b, int mode, int order) {
+  const int sp = order & HOP_SPATIAL;
+  if (mode == 2 && sitewave_ok(L, P, b, sp != 0)) return HOP_SITEWAVE | sp;
+  if (mode == 3 && lds_links_ok(P, b)) return HOP_LDS_LINKS | sp;
+  P.flags = HOP_LINK_ROW;
+  if (mode == 5 && link_row_setup(P, b)) return HOP_LINK_ROW | sp;
+  if (mode == 4)
+    for (int G : {4, 2, 8, 16}) {
+      const int f = HOP_RHSGROUP | (__builtin_ctz(G / 2) << 6);
+      if (rhsgroup_ok(P, b, f | HOP_SPATIAL)) return f | HOP_SPATIAL;
+      if (rhsgroup_ok(P, b, f)) return f;
+    }
+  return order;
+}
+
 // CPS_HIP_TUNE_REPORT=1 prints each tuning decision to stderr, =2 also the
 // time of every candidate
 static int tune_report() { return knob(&cps_hip_tuning::tune_report, "CPS_HIP_TUNE_REPORT"); }
@@ -630,6 +649,9 @@ int tuned_launch(Lattice& L, HopParams& P) {
   }
   HopTuneKey key{P.kind, P.prec, P.dag, P.nb, P.nsites_out, P.nrhs, P.partial != nullptr, P.X.data != nullptr,
                  P.clov + 16 * P.m5post + 32 * P.rupd, {L.g.L[0], L.g.L[1], L.g.L[2], L.g.L[3]}, mode + (quad ? 16 : 0)};
+  // a launch that updates a field in place (rupd) is never timed on the live
+  // data: it keeps the order of order_rule or rupd_rule
+  const bool timed = tuning_enabled() && !P.rupd;
   HopTuneVal chosen;
   bool have = false;
   {
@@ -652,7 +674,7 @@ int tuned_launch(Lattice& L, HopParams& P) {
     // order in every mapping, so a rhs-group choice that the count no
     // longer allows falls back to element order)
     for (const auto& kv : tune_cache) {
-      if (P.rupd) break;   // never timed: its rule is cheap and follows the count
+      if (!timed) break;   // the rules are cheap and follow the count
       HopTuneKey k2 = kv.first;
       k2.nrhs = key.nrhs;
       if (k2 < key || key < k2) continue;
@@ -670,15 +692,15 @@ int tuned_launch(Lattice& L, HopParams& P) {
   }
   if (!have) {
     HopTuneVal best{def_block, order_rule(L, P, def_block, quad), 0.0};
-    // a launch that updates a field in place (rupd) is never timed on the
-    // live data: it keeps the order of order_rule or rupd_rule
-    if (P.rupd) {
-      rupd_rule(P, mode, best);
+    if (!timed) {
+      if (P.rupd) rupd_rule(P, mode, best);
+      else best.flags = mapping_rule(L, P, def_block, mode, best.flags);
       if (tune_report() >= 1)
-        fprintf(stderr, "cps_hip rule: kind %d prec %d dag %d nb %d nsites %d nrhs %d clov %d residual step -> block %d flags %d\n",
-                P.kind, P.prec, P.dag, P.nb, P.nsites_out, P.nrhs, P.clov, best.block, best.flags);
+        fprintf(stderr, "cps_hip rule: kind %d prec %d dag %d nb %d nsites %d nrhs %d clov %d%s -> block %d flags %d\n",
+                P.kind, P.prec, P.dag, P.nb, P.nsites_out, P.nrhs, P.clov, P.rupd ? " residual step" : "", best.block,
+                best.flags);
     }
-    if (tuning_enabled() && !P.rupd) {
+    if (timed) {
       std::vector<int> blocks;
       if (P.partial && !hop_chunk_partials(P)) blocks.push_back(def_block);
       else
