@@ -25,6 +25,13 @@ static hipError_t launch_c(const HopParams& P, hipStream_t st) {
   if (per_rhs % bs && (P.flags & (HOP_SPATIAL | HOP_LDS_LINKS)) &&
       !(P.flags & (HOP_SITEWAVE | HOP_RHSGROUP)))
     return hipErrorInvalidValue;
+  // the spatial order: its table, and whole blocks (or sites of a block) per
+  // spatial block, dealt to the XCDs in ranges
+  if (P.flags & HOP_SPATIAL) {
+    const int64_t per_b = (P.flags & HOP_SITEWAVE) ? (int64_t)P.perm_S * 64 : (int64_t)P.perm_S * P.nb;
+    if (!P.perm || (P.flags & HOP_NO_XCD_REMAP) || (!(P.flags & HOP_RHSGROUP) && per_b % bs))
+      return hipErrorInvalidValue;
+  }
   int64_t nblk = (int64_t)block_count(per_rhs, bs) * P.nrhs;
   if (P.flags & HOP_RHSGROUP) {
     // rhs groups times blocks of W S sites

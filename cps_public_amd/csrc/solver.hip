@@ -663,7 +663,9 @@ int tuned_launch(Lattice& L, HopParams& P) {
     }
   }
   // the spatial order's table, built on the handle's first use of it
-  if ((!have || (chosen.flags & HOP_SPATIAL)) && L.perm_state >= 0 && L.g.Vcb % 8 == 0 && L.ensure_perm() == 0)
+  int perm_rc = CPS_HIP_ERR_ARG;
+  if ((!have || (chosen.flags & HOP_SPATIAL)) && L.perm_state >= 0 && L.g.Vcb % 8 == 0 &&
+      (perm_rc = L.ensure_perm()) == 0)
     P.perm = (const uint32_t*)(P.kind == KIND_DWF ? L.perm5.p : L.perm.p);
   if (!have) {
     std::lock_guard<std::mutex> lk(tune_mu);
@@ -787,6 +789,8 @@ int tuned_launch(Lattice& L, HopParams& P) {
     std::lock_guard<std::mutex> lk(tune_mu);
     tune_cache.emplace(key, best);
   }
+  // (a handle whose table could not be allocated, where another one's could)
+  if ((chosen.flags & HOP_SPATIAL) && !P.perm) return perm_rc;
   P.block = chosen.block;
   P.flags = chosen.flags;
   CPSHIP_CHECK(launch_hop(P, L.stream));
