@@ -113,7 +113,7 @@ int Lattice::set_twist(const double angle[4]) {
 
 long long Lattice::device_bytes() const {
   long long b = (long long)gauge_aos.bytes + partial.bytes + scal.bytes + io.bytes + io2.bytes + nbr.bytes +
-                nbr_neg.bytes + det_scratch.bytes + gauge_stage.bytes;
+                nbr_neg.bytes + perm.bytes + perm5.bytes + clover_ksq.bytes + det_scratch.bytes + gauge_stage.bytes;
   for (int k = 0; k < NLINK; k++) b += gauge[k].bytes;
   for (auto& f : scratch) b += f.buf.bytes + f.nrm.bytes;
   for (int k = 0; k < NCLOVER; k++) b += clover[k].bytes;

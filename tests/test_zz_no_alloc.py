@@ -71,3 +71,17 @@ def test_noalloc_matches_spatial_order(L, ls):
     lat.close()
     assert np.array_equal(first, ref) and np.array_equal(again, ref)
     assert np.array_equal(dfirst, dref) and np.array_equal(dagain, dref)
+
+
+def test_spatial_order_tables_are_counted():
+    """The site tables of the spatial order (4 bytes a site of one parity, and
+    4 of both for domain-wall fields), built with a handle of Ls 16, are in
+    its device bytes."""
+    L = [4, 4, 4, 8]
+    vcb = int(np.prod(L)) // 2
+    size = {}
+    for ls in (8, 16):
+        lat = C.Lattice(L, ls, (0, 0, 0, 1))
+        size[ls] = lat.device_bytes()
+        lat.close()
+    assert size[16] - size[8] == 4 * vcb + 8 * vcb
