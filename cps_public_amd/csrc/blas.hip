@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(256) k_cg_xr_t(FieldRef x, FieldRef p, FieldRe
   block_partial_d(in ? n : 0.0, partial, slot);
 }
 
-// The mixed CG's lagged solution update: the step x += alpha p of the
+// The lagged solution update (FP64 and mixed CG): the step x += alpha p of the
 // previous iteration is applied by the kernel that reads p next, the
 // direction update p = r + beta p (alpha[rhs] = 0 when no step is pending;
 // a rhs that stopped still gets its last step, but no new direction).

@@ -87,9 +87,10 @@ struct Lattice {
   DevBuf partial, scal, io, io2;
   HostStager stager;   // large copies from and to the caller's host vectors
   DevBuf nbr, nbr_neg;   // neighbour table of the geometry (hop kernels)
-  // spatial site order of the HOP_SPATIAL launches (built on first use),
-  // perm for one parity and perm5 for both (DWF fields): 0 not built, 1
-  // built, -1 the geometry has no 8-way (y, z) split
+  // spatial site order of the HOP_SPATIAL launches (built with the handle
+  // from Ls 16 on, else on first use), perm for one parity and perm5 for both
+  // (DWF fields): 0 not built, 1 built, -1 the geometry has no 8-way (y, z)
+  // split
   DevBuf perm, perm5;
   int perm_state = 0;
   int ensure_perm();

@@ -108,14 +108,14 @@ typedef struct {
  * overrides the field of the same name.  No counterpart in CPS. */
 typedef struct {
   int use_graph;        /* 1: CG iterations replayed as a captured hipGraph (ANDed with cps_hip_cg_arg.use_graph) */
-  int tune;             /* 1: the hop autotuner times its candidates; 0: default launch */
-  int tune_report;      /* 1: print the tuner's choices, 2: also every candidate's time */
-  int hop_mode;         /* restrict the hop's thread mapping: 0 any, 1 element, 2 sitewave, 3 lds, 4 rhsgroup, 5 row-shared links (only reachable this way) */
+  int tune;             /* 1: the hop autotuner times its candidates; 0: default launch in the mapping of hop_mode */
+  int tune_report;      /* 1: print the launch choices (the tuner's, and those made by rule), 2: also every candidate's time */
+  int hop_mode;         /* restrict the hop's thread mapping: 0 any, 1 element, 2 sitewave, 3 lds, 4 rhsgroup, 5 row-shared links (only reachable this way); any value but 0 also keeps half precision off the matrix-core mapping */
   int rhs_window;       /* 1: kernels run on the contiguous range of rhs still iterating */
-  int lagged_x;         /* mixed CG: solution step applied by the next direction update */
+  int lagged_x;         /* CG, FP64 and mixed: solution step applied by the next direction update; 0 also turns r_in_hop and clover_r_in_hop off */
   int paired_x;         /* mixed CG: two solution steps per pass over x (FP16 directions) */
   int s5_xpay;          /* mixed Moebius Ls 16: first fifth-dimension step of M in the direction update */
-  int r_in_hop;         /* mixed Moebius Ls 16 and DWF: residual step in the last hop of M^dag (rounds differently) */
+  int r_in_hop;         /* residual step in the last kernel of M^dag: Wilson and DWF, FP64 and half precision; Moebius in half precision, Ls 16 or an Ls that does not divide 64 (rounds differently: FP64 in the order of the |r|^2 sum only) */
   int clover_r_in_hop;  /* mixed clover: residual step in the last hop of MatPcDag (default 0: it spills) */
   int m5_fused;         /* half precision Ls 16: M5^-1 in the first hop's epilogue */
   int s5_fused;         /* Moebius M^dag: last fifth-dimension step in the hop epilogue */

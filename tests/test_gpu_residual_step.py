@@ -84,3 +84,47 @@ def test_residual_step_mappings(monkeypatch, capfd, L, nrhs):
     for k in range(nrhs):
         part = slice(24 * n * k, 24 * n * (k + 1))
         assert rel(xg[part], xe[part]) < 2e-8
+
+
+@pytest.mark.parametrize("kind", ["wilson", "dwf", "mobius", "clover"])
+@pytest.mark.parametrize("graph", [1, 0])
+def test_fp64_lagged_steps(monkeypatch, kind, graph):
+    """FP64 solves whose rhs converge at different iterations (the first and
+    the last start close to their solutions, so the window of active rhs
+    shrinks at both ends, where pending solution steps are applied).
+    CPS_HIP_LAGGED_X=0 with the residual step a pass of its own: the same
+    arithmetic, so the same bits.  CPS_HIP_R_IN_HOP=0: the same for the
+    operators without that step; for Wilson and domain wall |r|^2 is the sum
+    of other partials, so twice the stopping rule's 1e-10 times the condition
+    of M^dag M (21 and 60 on these fields), and the iterations to one."""
+    L, nrhs, kappas = [4, 4, 4, 8], 4, [0.130, 0.1325]
+    ls = 8 if kind in ("dwf", "mobius") else 1
+    op = {"wilson": C.make_op(C.OP_WILSON, mass=0.1), "dwf": C.make_op(C.OP_DWF, mass=0.1, m5=1.8),
+          "mobius": C.make_op(C.OP_MOBIUS, mass=0.1, m5=1.8, b=1.5, c=0.5),
+          "clover": C.make_op(C.OP_CLOVER, mass=1.0 / (2 * kappas[0]) - 4.0, csw=1.0)}[kind]
+    n = int(np.prod(L)) // 2 * ls
+    src = np.concatenate([F.gaussian_fermion(n, 91 + k) for k in range(nrhs)])
+    lat = C.Lattice(L, ls, (0, 0, 0, 1))
+    lat.import_gauge(wilson_gauge(L, 0.2, 90))
+    if kind == "clover":
+        lat.clover_build(kappas, 1.0)
+    guess = np.zeros_like(src)
+    near, _ = lat.invcg(op, src, C.make_cg_arg(1e-5, 1000), nrhs=nrhs)
+    for k in (0, nrhs - 1):
+        guess[24 * n * k:24 * n * (k + 1)] = near[24 * n * k:24 * n * (k + 1)]
+    arg = C.make_cg_arg(1e-10, 1000)
+    arg.check_every, arg.use_graph = 3, graph
+    out = {}
+    for lagged, in_hop in (("1", "1"), ("1", "0"), ("0", "0"), ("0", "1")):
+        monkeypatch.setenv("CPS_HIP_LAGGED_X", lagged)
+        monkeypatch.setenv("CPS_HIP_R_IN_HOP", in_hop)
+        x, res = lat.invcg(op, src, arg, guess=guess, nrhs=nrhs)
+        out[lagged + in_hop] = (x, [r.iterations for r in res], max(r.true_res for r in res))
+    lat.close()
+    x, its, _ = out["00"]
+    assert max(its[0], its[-1]) + 3 < min(its[1:-1])
+    assert max(o[2] for o in out.values()) <= 1.1e-10
+    for same in ("10", "01") + (("11",) if kind in ("mobius", "clover") else ()):
+        assert np.array_equal(out[same][0], x) and out[same][1] == its
+    assert all(abs(a - b) <= 1 for a, b in zip(out["11"][1], its))
+    assert all(rel(out["11"][0][p], x[p]) < 1.2e-8 for p in (slice(24 * n * k, 24 * n * (k + 1)) for k in range(nrhs)))
