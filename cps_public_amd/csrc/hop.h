@@ -151,6 +151,7 @@ enum { CLOV_NONE = 0, CLOV_POST = 1, CLOV_X = 2, CLOV_S5X = 3, CLOV_S5XR = 4, CL
 
 hipError_t launch_hop(const HopParams& P, hipStream_t st);
 hipError_t build_nbr(const Geom& g, uint4* nbr, uint32_t* nbr_neg, hipStream_t st);
+hipError_t build_perm(const Geom& g, int by, int bz, uint32_t* perm, uint32_t* perm5, hipStream_t st);
 hipError_t launch_hop_clover(const HopParams& P, hipStream_t st);
 hipError_t launch_hop_quad(const HopParams& P, hipStream_t st);
 hipError_t pack_gauge_quad(bool bf16, const double* aos, void* out, const uint4* nbr, int Vcb, hipStream_t st);

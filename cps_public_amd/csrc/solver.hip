@@ -92,11 +92,11 @@ int Lattice::init(const int node_sites[4], int ls_, const int bc[4]) {
   if (rc) return rc;
   if ((rc = nbr_neg.ensure((size_t)2 * g.Vcb * sizeof(uint32_t)))) return rc;
   CPSHIP_CHECK(build_nbr(g, (uint4*)nbr.p, (uint32_t*)nbr_neg.p, stream));
-  CPSHIP_CHECK(hipStreamSynchronize(stream));
   // domain-wall hops with partials are swept in the spatial order from Ls 16
   // on (order_rule), also by the call that may not allocate: its table is
   // there from the start (the handle's first hop would build it otherwise)
   if (ls >= 16 && ls % 2 == 0 && g.Vcb % 8 == 0 && (rc = ensure_perm()) && perm_state >= 0) return rc;
+  CPSHIP_CHECK(hipStreamSynchronize(stream));
   return 0;
 }
 
@@ -258,30 +258,10 @@ int Lattice::ensure_perm() {
     perm_state = -1;
     return CPS_HIP_ERR_ARG;
   }
-  const int lh = g.L[0] / 2, ny = g.L[1] / best_by, nz = g.L[2] / best_bz;
-  std::vector<uint32_t> h((size_t)g.Vcb);
-  size_t q = 0;
-  for (int bz = 0; bz < best_bz; bz++)
-    for (int by = 0; by < best_by; by++)
-      for (int t = 0; t < g.L[3]; t++)
-        for (int z = bz * nz; z < (bz + 1) * nz; z++)
-          for (int y = by * ny; y < (by + 1) * ny; y++)
-            for (int xh = 0; xh < lh; xh++) h[q++] = (uint32_t)(xh + lh * (y + g.L[1] * (z + g.L[2] * t)));
-  int rc = perm.ensure(h.size() * sizeof(uint32_t));
+  int rc = perm.ensure((size_t)g.Vcb * sizeof(uint32_t));
   if (rc) return rc;
-  CPSHIP_CHECK(hipMemcpy(perm.p, h.data(), h.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-  if (ls > 1) {
-    // both parities of a block's slice after one another
-    std::vector<uint32_t> h5(2 * h.size());
-    const size_t slice = (size_t)lh * ny * nz;
-    for (size_t k = 0; k < h.size() / slice; k++)
-      for (size_t i = 0; i < slice; i++) {
-        h5[2 * k * slice + i] = h[k * slice + i];
-        h5[(2 * k + 1) * slice + i] = (uint32_t)g.Vcb + h[k * slice + i];
-      }
-    if ((rc = perm5.ensure(h5.size() * sizeof(uint32_t)))) return rc;
-    CPSHIP_CHECK(hipMemcpy(perm5.p, h5.data(), h5.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-  }
+  if (ls > 1 && (rc = perm5.ensure((size_t)2 * g.Vcb * sizeof(uint32_t)))) return rc;
+  CPSHIP_CHECK(build_perm(g, best_by, best_bz, (uint32_t*)perm.p, ls > 1 ? (uint32_t*)perm5.p : nullptr, stream));
   perm_state = 1;
   return 0;
 }
