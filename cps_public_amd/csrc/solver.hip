@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 namespace cpship {
@@ -536,33 +537,54 @@ static std::map<HopTuneKey, HopTuneVal> tune_cache;
 
 // Launch of a residual step without a clover term (CLOV_NRR), in the mapping
 // that hop_mode asks for where there is one (the site-per-wavefront, LDS and
-// row mappings have no residual step).  One element per site: from 2^18
-// elements on the rhs groups, which share link loads that no cache holds by
-// then (FP64 16^3x32 Wilson, 12 rhs: G = 4 146, 2 172, element order 245 us);
-// below it blocks dealt over the XCDs in hardware order (10x12x14x18, 12 rhs:
-// 52 us against 60 in XCD ranges and 55 in groups), of one wavefront where
-// larger ones would leave CUs idle.  (Chunk partials: block partials, as a
-// domain-wall field of two slices has with one element per site too, are tied
-// to the default block.)  FP64 residuals that do not stay in the 256 MB cache
-// between two kernels are stored around it.
+// row mappings have no residual step).  One element per site, Wilson, us:
+//  - up to 3 2^14 elements blocks of one wavefront, where larger ones leave CUs
+//    idle (8^4, 12 rhs: FP64 10.8, half 5.8 against 12.4 and 6.0 in blocks of
+//    256; 12x12x6x12, 12 rhs, 62208 elements: 24.9 and 8.0 against 20.7, 7.2),
+//    up to 2^15 dealt over the XCDs in hardware order (8^3x16, 8 rhs: 11.5
+//    against 12.5 in XCD ranges; 12^4, 4 rhs, 41472 elements: 18.7 against
+//    14.7);
+//  - above it FP64 takes the rhs groups, which share link loads (against
+//    blocks of 256 in hardware order and in XCD ranges: 12^4, 6 rhs 21 against
+//    25, 25; 16x8x14x22, 6 rhs 39 against 53, 53, 8 rhs 38 against 64, 57;
+//    16^3x32, 12 rhs 177 against 386, 261; the other way round at 10x12x14x18,
+//    12 rhs: 64 against 57, 65);
+//  - of the group shapes the first whose blocks the 8 XCDs share equally, since
+//    only those are dealt in ranges of sites (G = 4, G = 2 in blocks of 128 and
+//    of 256: 12^3x24, 12 rhs 76, 63, 78; 16x8x14x22, 4 rhs 27, 20, 27);
+//  - half precision from 2^18 elements on as FP64 (16^3x32, 12 rhs: groups 40
+//    against 54 and 60, 4 rhs 16 against 19 and 22), from 2^16 on where the
+//    groups are dealt in ranges (16x8x14x22, 8 rhs 12 against 18, 15; 12^3x24,
+//    12 rhs 17 against 26, 26; the other way round at 16^4, 6 rhs: 14 against
+//    12, 17), else in hardware order (10x12x14x18, 12 rhs 14 against 16 in
+//    groups; 14^4, 12 rhs 19 against 22);
+//  - XCD ranges where no group divides the rhs (24^3x48, 3 rhs: FP64 405, half
+//    68 against 443, 96 in hardware order; FP64 16^3x32, 3 rhs: 72 against 79).
+// (Chunk partials: block partials, as a domain-wall field of two slices has
+// with one element per site too, are tied to the default block.)  FP64
+// residuals above 32 MiB are stored with streaming stores: 0-1% faster at all
+// sizes above, within the noise below.
 static void rupd_rule(const HopParams& P, int mode, HopTuneVal& best) {
   if (P.clov != CLOV_NONE) return;
   const int64_t n = (int64_t)P.nsites_out * P.nb * P.nrhs;
   if (hop_chunk_partials(P)) {
-    const bool small = n < (1 << 18);
-    if (small) {
-      if (n < 256 * 256) best.block = 64;
-      best.flags = HOP_NO_XCD_REMAP;
-    }
-    if (mode == 4 || (mode != 1 && !small))
-      for (int G : {4, 2}) {
-        const int f = HOP_RHSGROUP | ((G >> 2) << 6);
-        const int b = mode == 4 ? 256 : best.block;   // (256: a chunk's wavefronts in one block for both G)
-        if (rhsgroup_ok(P, b, f)) {
-          best.block = b;
-          best.flags = f;
-          break;
-        }
+    const bool tiny = n <= (3 << 14);
+    const bool small = tiny || (P.prec != PREC_D_D18 && n < (1 << 18));
+    if (tiny) best.block = 64;
+    if (small && !(tiny && n > (1 << 15))) best.flags = HOP_NO_XCD_REMAP;
+    const bool any = mode == 4 || (mode != 1 && !small);
+    const bool ranges = any || (mode != 1 && n > (1 << 16));
+    bool found = false;
+    for (int pass = ranges ? 0 : 2; pass < 2 && !found; pass++)
+      for (const auto& c : {std::pair<int, int>{4, 256}, {2, 256}, {2, 128}}) {
+        const int G = c.first, b = c.second, f = HOP_RHSGROUP | ((G >> 2) << 6);
+        if (!rhsgroup_ok(P, b, f)) continue;
+        const int64_t blocks = (int64_t)block_count((int64_t)P.nsites_out * P.nb, b / G) * (P.nrhs / G);
+        if (pass == 0 ? blocks % 8 != 0 : !any || b != 256) continue;
+        best.block = b;
+        best.flags = f;
+        found = true;
+        break;
       }
   }
   if (P.prec == PREC_D_D18 && n * 192 > (int64_t(32) << 20)) best.flags |= HOP_NT_STORE;
@@ -629,9 +651,6 @@ int tuned_launch(Lattice& L, HopParams& P) {
   }
   HopTuneKey key{P.kind, P.prec, P.dag, P.nb, P.nsites_out, P.nrhs, P.partial != nullptr, P.X.data != nullptr,
                  P.clov + 16 * P.m5post + 32 * P.rupd, {L.g.L[0], L.g.L[1], L.g.L[2], L.g.L[3]}, mode + (quad ? 16 : 0)};
-  // a launch that updates a field in place (rupd) is never timed on the live
-  // data: it keeps the order of order_rule or rupd_rule
-  const bool timed = tuning_enabled() && !P.rupd;
   HopTuneVal chosen;
   bool have = false;
   {
@@ -642,6 +661,9 @@ int tuned_launch(Lattice& L, HopParams& P) {
       have = true;
     }
   }
+  // a launch that updates a field in place (rupd) is never timed on the live
+  // data: it keeps the order of order_rule or rupd_rule
+  const bool timed = !have && !P.rupd && tuning_enabled();
   // the spatial order's table, built on the handle's first use of it
   int perm_rc = CPS_HIP_ERR_ARG;
   if ((!have || (chosen.flags & HOP_SPATIAL)) && L.perm_state >= 0 && L.g.Vcb % 8 == 0 &&

@@ -47,14 +47,14 @@ def _flags(err):
 RHSGROUP = 32   # HOP_RHSGROUP
 
 
-@pytest.mark.parametrize("L,nrhs", [([4, 4, 8, 4], 4), ([6, 6, 4, 6], 2), ([10, 4, 6, 6], 4), ([6, 10, 6, 6], 6),
-                                    ([14, 14, 10, 14], 14)])
+@pytest.mark.parametrize("L,nrhs", [([4, 4, 8, 4], 4), ([8, 8, 4, 4], 4), ([6, 6, 4, 6], 2), ([10, 4, 6, 6], 4),
+                                    ([6, 6, 6, 6], 4), ([6, 10, 6, 6], 6), ([14, 14, 10, 14], 14)])
 def test_residual_step_mappings(monkeypatch, capfd, L, nrhs):
     """Wilson solves with the hops, the residual step among them, in element
     order and with 4 or 2 rhs of a site in a wavefront (CPS_HIP_HOP_MODE):
-    whole and part chunks of 64 sites (256, 432, 720, 1080 and 13720 sites a
-    parity), rhs counts that 4 and that only 2 divides, the last one large
-    enough for streaming stores.  FP64: an element's arithmetic and the tree
+    whole and part chunks of 64 sites (256, 512, 432, 720, 648, 1080 and 13720
+    sites a parity), groups in blocks of 256 (4 and 2 rhs) and of 128 (the first
+    and the fourth case), the last one large enough for streaming stores.  FP64: an element's arithmetic and the tree
     of the partial sums are the same, so are all bits.  Half precision: the
     two mappings are separate compilations (a few FP32 results round
     differently), so twice the stopping rule's 1e-10 times the condition of
