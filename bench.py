@@ -353,6 +353,15 @@ def serve_stream(a):
     print(json.dumps(line))
 
 
+def hop_kernel(cfg, prec):
+    """The kernel that the hop of this workload runs in: half precision with a
+    multiple of 4 slots per site (Ls / 2 of a domain-wall field, the Ls slices
+    of a Moebius one) has a kernel of its own on the matrix cores."""
+    slots = {C.OP_DWF: cfg["ls"] // 2, C.OP_MOBIUS: cfg["ls"]}.get(cfg["kind"], 1)
+    name = "k_hop_quad" if prec in (C.PREC_MIXED_HALF, C.PREC_MIXED_BF16) and slots % 4 == 0 else "k_hop"
+    return name + (" (5-D DWF)" if cfg["kind"] == C.OP_DWF else " (4-D, batched)")
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -528,7 +537,7 @@ def main():
         "speedup_vs_fp64": (fp64["s_per_rhs"] / s_per_rhs) if fp64 else None,
         "err_vs_fp64": err64,
         "bf16_links": bf16,
-        "dslash": {"kernel": "k_hop (5-D DWF)" if cfg["kind"] == C.OP_DWF else "k_hop (4-D, batched)",
+        "dslash": {"kernel": hop_kernel(cfg, prec_main),
                    "seconds_per_launch": sec, "algorithmic_bytes": byt, "GBps": achieved,
                    "fp64_GBps": byt64 / sec64 / 1e9, "fp64_seconds_per_launch": sec64},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -21,11 +21,15 @@
 // the product uses.
 //
 // The element kernel issues ~900 vector instructions per wavefront here and
-// keeps the vector ALUs 55-60% busy; this one issues ~570 (64 of the
-// matrix instructions beside them) and is bound by the vector L1's outstanding misses
-// (60-80 lines per CU at 300-400 cycles, 11 TB/s over the chip): one hop of
-// the 16^3x32 lattice takes 452 instead of 488 us (Moebius, Ls 16, 12 rhs)
-// and, with the sites swept block by block (HOP_SPATIAL), 38 instead of 46 us
+// keeps the vector ALUs 55-60% busy; this one issues ~570 and 64 matrix
+// instructions, and is bound by the vector L1's data return and outstanding
+// misses: with the field in HBM the return path is busy 97% of the launch and
+// a CU has 59-82 lines in flight at 450-640 clocks, 10 TB/s from L2 over the
+// chip (16^3x32, Moebius, Ls 16, 12 rhs); with one rhs of a domain-wall field
+// 49-57 lines at 315-420 clocks while the CUs are busy 77-82% of a launch of
+// 36-55 us (profiles/performance_cases_hop_counters.txt).  One hop of the
+// 16^3x32 lattice takes 452 instead of 488 us (Moebius, Ls 16, 12 rhs) and,
+// with the sites swept block by block (HOP_SPATIAL), 38 instead of 46 us
 // (domain wall, Ls 16, 1 rhs).
 //
 // Neighbour loads run CPSHIP_QUAD_AHEAD directions ahead of the arithmetic:
