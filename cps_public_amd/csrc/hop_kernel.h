@@ -104,7 +104,11 @@ __device__ __forceinline__ void su3_dag_mul(const cplx<R> u[9], const cplx<R> h[
 // every neighbour 8 times from L2.  4-D kind: +mu, -mu in turn (FP64 Wilson
 // hop of 16^3x32, 12 rhs, 131 -> 115 us; +x +y -x -y ..: 121).  Domain-wall
 // kind, whose sites are 8 lanes wide: +x +y -x -y, +z +t -z -t (FP64,
-// 16^3x32, Ls 16: 189 -> 166 us; the other order 170).
+// 16^3x32, Ls 16: 189 -> 166 us; the other order 170).  Half precision and
+// FP32 gain less, whole solves against all +mu before all -mu: clover 24^3x48,
+// 8 rhs 202 -> 197 ms, Wilson 16^3x32, 12 rhs 35.0 -> 34.3, FP32 domain wall
+// 12^3x16, Ls 12, 4 rhs 62.6 -> 61.5; launches of a few 10^4 elements lose 2%
+// (clover 12x12x6x12, 5 rhs 12.3 -> 12.6).
 template <int KIND>
 __host__ __device__ constexpr int hop_dir(int k) {
   return KIND == KIND_DWF ? (k & 1) + (k & 2) * 2 + (k & 4) / 2 : (k >> 1) + 4 * (k & 1);
@@ -422,8 +426,8 @@ __device__ __forceinline__ void hop_batch(const HopParams& P, const Nbr& N, int 
   }
 #define CPSHIP_DIR(K)                                                                             \
   if constexpr ((K) < NB) {                                                                       \
-    const float2 ph = link_phase(P, N.neg, hop_dir<KIND>(D0 + (K)));                                             \
-    dir_compute<hop_dir<KIND>(D0 + (K)), SIN, LK, R, DAG>(sr[K], lr[K], ph, acc);                                \
+    const float2 ph = link_phase(P, N.neg, hop_dir<KIND>(D0 + (K)));                              \
+    dir_compute<hop_dir<KIND>(D0 + (K)), SIN, LK, R, DAG>(sr[K], lr[K], ph, acc);                 \
   }
   CPSHIP_DIR(0) CPSHIP_DIR(1) CPSHIP_DIR(2) CPSHIP_DIR(3) CPSHIP_DIR(4) CPSHIP_DIR(5) CPSHIP_DIR(6) CPSHIP_DIR(7)
 #undef CPSHIP_DIR
@@ -443,7 +447,7 @@ __device__ __forceinline__ void hop_lds_compute(const HopParams& P, const uint32
                                                 const SpinRaw<SpinH> sr[NB], cplx<float> acc[12]) {
 #define CPSHIP_DIR(K)                                                                             \
   if constexpr ((K) < NB) {                                                                       \
-    constexpr int D = hop_dir<KIND>(D0 + (K));                                                                 \
+    constexpr int D = hop_dir<KIND>(D0 + (K));                                                    \
     const uint4* w = reinterpret_cast<const uint4*>(lds + sl * LDS_SITE_WORDS + 8 * D);           \
     const uint4 a = w[0], b = w[1];                                                               \
     const uint32_t U[9] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w,                                \
@@ -840,10 +844,10 @@ __device__ __forceinline__ void hop_batch_row(const HopParams& P, const Nbr& N, 
   }
 #define CPSHIP_DIR(K)                                                                             \
   if constexpr ((K) < NB) {                                                                       \
-    const float2 ph = link_phase(P, N.neg, hop_dir<KIND>(D0 + (K)));                                             \
+    const float2 ph = link_phase(P, N.neg, hop_dir<KIND>(D0 + (K)));                              \
     uint32_t U[9];                                                                                \
     link_words_f16<LK>(link_from_row<LK>(lw[K]), ph, U);                                          \
-    dir_compute_h2w<hop_dir<KIND>(D0 + (K)), DAG>(sr[K], U, acc);                                                \
+    dir_compute_h2w<hop_dir<KIND>(D0 + (K)), DAG>(sr[K], U, acc);                                 \
   }
   CPSHIP_DIR(0) CPSHIP_DIR(1) CPSHIP_DIR(2) CPSHIP_DIR(3) CPSHIP_DIR(4) CPSHIP_DIR(5) CPSHIP_DIR(6) CPSHIP_DIR(7)
 #undef CPSHIP_DIR

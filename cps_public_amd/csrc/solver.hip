@@ -383,15 +383,15 @@ int hop_ex(Lattice& L, const cps_hip_op* op, int hprec, const FieldRef& out, con
 // ---------------------------------------------------------------------------
 // Autotuner: the first launch of each hop shape (kind, precision, dag, batch,
 // volume, rhs count, epilogue) times every candidate block size and launch
-// variant on the real operands and keeps the fastest for the lattice
-// handle's lifetime.  Launches that write per-block reduction partials keep
-// the default block size, because the reduction reads one partial per block;
-// per-chunk partials (4-D operators) are summed in an order that does not
-// depend on the block or mapping.  The candidates compute every element with
-// the same source arithmetic: FP64 results are the same bits whichever wins;
-// the half-precision kernels of different mappings are separate compilations
-// and may round a few FP32 results differently (FMA contraction).
-// CPS_HIP_TUNE=0 switches tuning off (default block, no variants).
+// variant on the real operands and keeps the fastest for the process.
+// Launches that write per-block reduction partials keep the default block
+// size, because the reduction reads one partial per block; per-chunk partials
+// (4-D operators) are summed in an order that does not depend on the block or
+// mapping.  The candidates compute every element with the same source
+// arithmetic: FP64 results are the same bits whichever wins; the half-
+// precision kernels of different mappings are separate compilations and may
+// round a few FP32 results differently (FMA contraction). CPS_HIP_TUNE=0
+// switches tuning off (default block, no variants).
 
 static std::mutex tuning_mu;
 static cps_hip_tuning tuning_fields = {1, 1, 0, 0, 1, 1, 1, 1, 1, 0, 1, 1, 1, 0, 0, 0.0};
